@@ -961,16 +961,14 @@ int mi355moe_moe_layer(const mi355moe_exl3_layer* layer, const void* x, int x_dt
     router_scratch(static_cast<char*>(workspace) + align_up((size_t)base), T, topk, E, &lg, &ids, &wts);
     if (ids_out) ids = ids_out;
     if (weights_out) wts = weights_out;
-    // router GEMV, top-k, then the routed experts from the picks
+    // router, top-k, then the routed experts from the picks
     const int64_t P = T * topk;
-    const bool small = choose_path(layer, P, MI355MOE_PATH_AUTO) == MI355MOE_PATH_DECODE && P <= ROUTE_SMALL_MAX_P;
+    // one launch ranks in its last workgroup: up to 24 tokens; beyond, the bounded logits with a wave per token (288
+    // experts, hidden 4096, whole layer: T = 16 208 against 215 us, 24 equal, 32 320 against 314, 64 444 against 420)
+    constexpr int64_t ONE_LAUNCH_T = 24;
+    const bool small = choose_path(layer, P, MI355MOE_PATH_AUTO) == MI355MOE_PATH_DECODE && P <= ROUTE_SMALL_MAX_P &&
+                       (!router_w || T <= ONE_LAUNCH_T);
     const float* lsrc = logits;
-    if (router_w && !small) {
-        if (int rc = launch_router_logits(static_cast<const uint16_t*>(x), x_stride,
-                                          static_cast<const uint16_t*>(router_w), (int)T, (int)K, (int)E, lg, stream))
-            return rc_launch(rc);
-        lsrc = lg;
-    }
     if (small) {
         // decode sizes: the router GEMV (when given the weight), the top-k and the permutation in one launch (the
         // last router workgroup ranks), then the expert GEMVs and the combine
@@ -995,9 +993,12 @@ int mi355moe_moe_layer(const mi355moe_exl3_layer* layer, const void* x, int x_dt
         if (rc) return rc_launch(rc);
         return rc_launch(launch_decode(w.da, p.rmax, stream, MI355MOE_STAGE_ALL >> 1));
     }
-    if (int rc = launch_router_topk(lsrc, (int)T, (int)E, bias, (int)topk, routed_scale, renormalize ? 1 : 0, ids, wts,
-                                    stream))
-        return rc_launch(rc);
+    const int rc = router_w ? launch_router_picks(static_cast<const uint16_t*>(x), x_stride,
+                                                  static_cast<const uint16_t*>(router_w), (int)T, (int)K, (int)E, lg,
+                                                  bias, (int)topk, routed_scale, renormalize ? 1 : 0, ids, wts, stream)
+                            : launch_router_topk(lsrc, (int)T, (int)E, bias, (int)topk, routed_scale,
+                                                 renormalize ? 1 : 0, ids, wts, stream);
+    if (rc) return rc_launch(rc);
     return mi355moe_moe_forward_ids_ex(layer, x, x_dtype, x_stride, T, ids, MI355MOE_I32, wts, MI355MOE_F32, topk,
                                        nullptr, 0, limit, out, out_dtype, out_stride, workspace, (size_t)base,
                                        MI355MOE_PATH_AUTO, MI355MOE_STAGE_ALL, stream);

@@ -277,6 +277,11 @@ int launch_router_logits(const uint16_t* x, int64_t x_stride, const uint16_t* w,
                          hipStream_t st);
 int launch_router_topk(const float* logits, int T, int E, const float* bias, int topk, float scale, int renorm,
                        int32_t* ids, float* wts, hipStream_t st);
+// the picks and weights of T tokens from the router's operands, without every logit's exact value (bounds: [T][E]
+// scratch); the same picks and weights as launch_router_logits and launch_router_topk
+int launch_router_picks(const uint16_t* x, int64_t x_stride, const uint16_t* w, int T, int K, int E, float* bounds,
+                        const float* bias, int topk, float scale, int renorm, int32_t* ids, float* wts,
+                        hipStream_t st);
 int launch_route(const RouteArgs& a, hipStream_t st);
 // segment tables of rows grouped by expert from int64 counts [n] (n <= 4096), ceil(count / tile) segments each
 int launch_seg_tables(const int64_t* counts, int n, int tile, int max_segs, int* se, int* sr0, int* sr, int* ns,

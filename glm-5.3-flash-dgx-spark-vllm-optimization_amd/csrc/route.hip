@@ -189,6 +189,219 @@ __global__ __launch_bounds__(256) void router_gemm_f64_kernel(const uint16_t* __
 }
 constexpr int RG_MIN_T = 256;   // from this many tokens the MFMA GEMM beats the GEMV kernel
 
+// Router logits for the top-k alone (router_bound_kernel, router_bound_big_kernel): products on the bf16 matrix cores
+// with fp32 sums, a rigorous bound on their error, and for every logit either its value (the bound leaves one bf16
+// value possible) or an upper bound of it; the top-k then takes the exact dot product of a candidate only when its
+// upper bound wins a round (topk_wave, LAZY): about one per token. The picks and weights are those of the exact logits.
+//
+// Error bound: a sum runs as chains of 64 products from zero, each chain added to an fp32 total (and the totals of a
+// workgroup's K ranges added in order). However the matrix core orders, aligns and truncates, an addend of an MFMA
+// loses at most 2^-23 of the chain's sum of |products|, so a chain (4 MFMAs of 16 products or 2 of 32, with their
+// accumulators at most 68 addends) is off by 68 * 2^-23 of it, and each of the K / 64 + 8 further additions by 2^-24 of
+// the whole: together (136 + K / 64 + 8) 2^-24 * sum of |x_k w_k|, itself at most |x| |w| (Cauchy-Schwarz; the norms
+// come from the same operands, 1 % added for their own rounding). T = 8192 tokens x 288 experts x 4096: bounds 63 us and
+// lazy top-k 37 us, against 525 us for every logit on the float64 matrix cores (37 TFLOP/s of 78) and 14 us for its
+// top-k; T = 64: 11 + 14 us, against 72 us for the one-launch front end.
+// Stored words: low half zero = the logit (a bf16 value); low half one = the high half is an upper bound (NaN where
+// nothing is known: sums or norms that overflow, underflow or are not finite).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ float sum_sq8(const u32x4& v, float s) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t u = v[i];
+        s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, u), __builtin_bit_cast(bf16x2, u), s, false);
+    }
+    return s;
+}
+// The stored word of a logit from its fp32 sum s and the operands' squared norms.
+__device__ __forceinline__ float bound_word(float s, float x2, float w2, int K) {
+    const float c = 1.01f * (float)(144 + (K >> 6)) * 5.9604645e-8f;
+    const float d = c * __builtin_sqrtf(x2) * __builtin_sqrtf(w2) + 4.8e-7f * fabsf(s);
+    const uint32_t lo = f32_to_bf16(s - d), hi = f32_to_bf16(s + d);
+    // norms whose squares lie outside the range where fp32 sums of them hold: nothing is known
+    const bool ok = x2 > 1e-25f && x2 < 1e25f && w2 > 1e-25f && w2 < 1e25f && fabsf(s) < 1e30f;
+    return __builtin_bit_cast(float, !ok ? 0x7FFF0001u : lo == hi ? lo << 16 : (hi << 16) | 1u);
+}
+
+// 16 tokens x 16 experts per workgroup, its eight waves an eighth of K each: a small call is bound by the latency of its
+// loads, so its tiles are small (72 workgroups for 64 tokens x 288 experts) and a wave's 32 loads of a 512-wide range
+// are all in flight before the first product. Lane (r = lane % 16, g = lane / 16) reads row r's bytes 16 g .. + 15 of
+// every 64 (whole 64-byte runs); both operands take the same k order.
+// ST: the 64-k steps whose loads are issued together, a divisor of a wave's K / 512 steps.
+constexpr int RB_WAVES = 8;
+template <int ST>
+__global__ __launch_bounds__(64 * RB_WAVES) void router_bound_kernel(const uint16_t* __restrict__ x, int64_t x_stride,
+                                                                     const uint16_t* __restrict__ w, int T, int K,
+                                                                     int E, float* __restrict__ bounds) {
+    __shared__ float cs[RB_WAVES][16 * 16], nx[RB_WAVES][16], nw[RB_WAVES][16];
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tiles_e = (E + 15) / 16;
+    const int t0 = ((int)blockIdx.x / tiles_e) * 16, e0 = ((int)blockIdx.x % tiles_e) * 16;
+    const int kr = K / RB_WAVES;                                     // a multiple of 64
+    const uint16_t* xp = x + (size_t)min(t0 + r, T - 1) * x_stride + wv * kr + 8 * g;
+    const uint16_t* wp = w + (size_t)min(e0 + r, E - 1) * K + wv * kr + 8 * g;
+    f32x4 tot = {0.f, 0.f, 0.f, 0.f};
+    float sx = 0.f, sw = 0.f;
+    for (int k0 = 0; k0 < kr; k0 += 64 * ST) {
+        u32x4 xa[ST][2], wa[ST][2];
+#pragma unroll
+        for (int s = 0; s < ST; ++s)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int k = k0 + 64 * s + 32 * j;
+                xa[s][j] = *reinterpret_cast<const u32x4*>(xp + k);
+                wa[s][j] = *reinterpret_cast<const u32x4*>(wp + k);
+            }
+        __builtin_amdgcn_sched_barrier(0);                           // every load issued before the first use
+#pragma unroll
+        for (int s = 0; s < ST; ++s) {
+            f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, xa[s][j]),
+                                                            __builtin_bit_cast(bf16x8, wa[s][j]), c, 0, 0, 0);
+                sx = sum_sq8(xa[s][j], sx);
+                sw = sum_sq8(wa[s][j], sw);
+            }
+            tot += c;
+        }
+    }
+    sx += xor_lane<16>(sx, lane);
+    sx += xor_lane<32>(sx, lane);
+    sw += xor_lane<16>(sw, lane);
+    sw += xor_lane<32>(sw, lane);
+    if (g == 0) {
+        nx[wv][r] = sx;
+        nw[wv][r] = sw;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) cs[wv][(4 * g + q) * 16 + r] = tot[q];   // D: column lane % 16, row 4 g + q
+    __syncthreads();
+    if (threadIdx.x >= 256) return;
+    const int row = (int)threadIdx.x >> 4, col = (int)threadIdx.x & 15;
+    float s = cs[0][threadIdx.x], x2 = nx[0][row], w2 = nw[0][col];
+#pragma unroll
+    for (int v = 1; v < RB_WAVES; ++v) {
+        s += cs[v][threadIdx.x];
+        x2 += nx[v][row];
+        w2 += nw[v][col];
+    }
+    if (t0 + row < T && e0 + col < E) bounds[(size_t)(t0 + row) * E + e0 + col] = bound_word(s, x2, w2, K);
+}
+
+// 64 tokens x 96 experts per workgroup (288 experts are three such tiles), four waves: wave (b, q) takes token block b of
+// 32 and the k half q of every 64-k step; the two halves' totals are added at the end. The tile's 160 operand rows are
+// staged 64 k (128 bytes a row) at a time by LDS DMA, three stages deep (60 KB, two workgroups per CU), chunk c of row R
+// at slot c ^ (R / 2 % 8) so that the fragment reads are free of bank conflicts. A large call reads every operand byte
+// once per tile instead of once per 16 rows. Wave (0, q) also squares expert blocks 0 and 1, wave (1, q) block 2.
+constexpr int RBB_TOK = 64, RBB_EXP = 96, RBB_NS = 3, RBB_STAGE = (RBB_TOK + RBB_EXP) * 128;
+constexpr int RBB_INST = (RBB_TOK + RBB_EXP) / 8 / 4;                 // DMA instructions per wave and stage
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void router_bound_big_kernel(
+    const uint16_t* __restrict__ x, int64_t x_stride, const uint16_t* __restrict__ w, int T, int K, int E,
+    float* __restrict__ bounds) {
+    __shared__ __align__(16) unsigned char lds[RBB_NS * RBB_STAGE];
+    const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = wv >> 1, q2 = wv & 1;
+    const int tiles_e = (E + RBB_EXP - 1) / RBB_EXP;
+    const int t0 = ((int)blockIdx.x / tiles_e) * RBB_TOK, e0 = ((int)blockIdx.x % tiles_e) * RBB_EXP;
+    const int steps = K >> 6;
+    const uint16_t* src[RBB_INST];
+#pragma unroll
+    for (int i = 0; i < RBB_INST; ++i) {
+        const int R = (RBB_INST * wv + i) * 8 + (lane >> 3);
+        const uint16_t* row = R < RBB_TOK ? x + (size_t)min(t0 + R, T - 1) * x_stride
+                                          : w + (size_t)min(e0 + R - RBB_TOK, E - 1) * K;
+        src[i] = row + 8 * ((lane & 7) ^ ((R >> 1) & 7));
+    }
+    auto issue = [&](int st) {
+        unsigned char* d = lds + (st % RBB_NS) * RBB_STAGE + RBB_INST * wv * 1024;
+        const int k = min(st, steps - 1) * 64;                       // (past the end: the last step again)
+#pragma unroll
+        for (int i = 0; i < RBB_INST; ++i) dma16(src[i] + k, d + i * 1024);
+    };
+    auto frag = [&](const unsigned char* st, int R, int j) {
+        return *reinterpret_cast<const u32x4*>(st + R * 128 + (((2 * j + h) ^ ((R >> 1) & 7)) << 4));
+    };
+    f32x16 tot[3];
+#pragma unroll
+    for (int n = 0; n < 3; ++n)
+#pragma unroll
+        for (int q = 0; q < 16; ++q) tot[n][q] = 0.f;
+    float sx[2] = {0.f, 0.f}, sw[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+#pragma unroll
+    for (int s = 0; s < RBB_NS - 1; ++s) issue(s);
+    for (int st = 0; st < steps; ++st) {
+        WAIT_VM(RBB_INST * (RBB_NS - 2));
+        LDS_BARRIER();
+        const unsigned char* d = lds + (st % RBB_NS) * RBB_STAGE;
+        u32x4 xa[2], wa[2][3];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            xa[j] = frag(d, 32 * b + r, 2 * q2 + j);
+#pragma unroll
+            for (int n = 0; n < 3; ++n) wa[j][n] = frag(d, RBB_TOK + 32 * n + r, 2 * q2 + j);
+        }
+        issue(st + RBB_NS - 1);
+        f32x16 c[3] = {};
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int n = 0; n < 3; ++n)
+                c[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xa[j]),
+                                                               __builtin_bit_cast(bf16x8, wa[j][n]), c[n], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            sx[j] = sum_sq8(xa[j], sx[j]);
+            if (b == 0) {                                            // (uniform)
+                sw[0][j] = sum_sq8(wa[j][0], sw[0][j]);
+                sw[1][j] = sum_sq8(wa[j][1], sw[1][j]);
+            } else {
+                sw[0][j] = sum_sq8(wa[j][2], sw[0][j]);
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < 3; ++n) tot[n] += c[n];
+    }
+    WAIT_VM(0);
+    LDS_BARRIER();                                                   // nothing in flight, every stage read
+    float* cs = reinterpret_cast<float*>(lds);                       // [block b][expert block][32][32] of the q = 1 waves
+    float* nx = cs + 2 * 3 * 1024;                                   // [q][64], [q][96]
+    float* nw = nx + 2 * RBB_TOK;
+    const float x2p = sx[0] + sx[1], w2p = sw[0][0] + sw[0][1], w2q = sw[1][0] + sw[1][1];
+    const float x2s = x2p + xor_lane<32>(x2p, lane), w2s = w2p + xor_lane<32>(w2p, lane),
+                w2t = w2q + xor_lane<32>(w2q, lane);
+    if (h == 0) {
+        nx[q2 * RBB_TOK + 32 * b + r] = x2s;
+        nw[q2 * RBB_EXP + 64 * b + r] = w2s;
+        if (b == 0) nw[q2 * RBB_EXP + 32 + r] = w2t;
+    }
+    // D: column lane % 32, row 8 (q / 4) + 4 h + q % 4
+    if (q2 == 1)
+#pragma unroll
+        for (int n = 0; n < 3; ++n)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) cs[((b * 3 + n) * 32 + 8 * (q >> 2) + 4 * h + (q & 3)) * 32 + r] = tot[n][q];
+    __syncthreads();
+    if (q2 == 1) return;
+#pragma unroll
+    for (int n = 0; n < 3; ++n) {
+        const int e = e0 + 32 * n + r;
+        const float w2 = nw[32 * n + r] + nw[RBB_EXP + 32 * n + r];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const int row = 8 * (q >> 2) + 4 * h + (q & 3), t = 32 * b + row;
+            const float s = tot[n][q] + cs[((b * 3 + n) * 32 + row) * 32 + r];
+            if (t0 + t < T && e < E) bounds[(size_t)(t0 + t) * E + e] = bound_word(s, nx[t] + nx[RBB_TOK + t], w2, K);
+        }
+    }
+}
+// Tokens from which the big tiles win (whole layer, 288 experts x 4096, big against small tiles: T = 300 621 / 607 us,
+// 600 905 / 903, 1024 875 / 877, 1791 961 / 977).
+constexpr int RB_BIG_T = 1024;
+
 __global__ __launch_bounds__(1024) void router_logits_kernel(const uint16_t* __restrict__ x, int64_t x_stride,
                                                              const uint16_t* __restrict__ w, int T, int K, int E,
                                                              float* __restrict__ logits) {
@@ -467,19 +680,61 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
 // reference's order). Scores s = sigmoid(logit)
 // (through double exp) go to sco [E] for the weights; weights are the picks' scores renormalised over their total
 // (summed sequentially in pick order, + 1e-20, correctly rounded division) and scaled.
-// J >= ceil(E / 64); COH: coherent loads of the row; SCORE: the row holds the scores sigmoid(logit) already
-template <int J, bool COH = false, bool SCORE = false>
+// J >= ceil(E / 64); COH: coherent loads of the row; SCORE: the row holds the scores sigmoid(logit) already. LAZY: the
+// row holds router_bound_kernel's words; a candidate known by its upper bound is ranked by it, and when it wins a round
+// its exact logit (the float64 dot product of xrow and its weight row) takes the bound's place and the round is run
+// again. Key and score grow with the logit, so a candidate that loses with its upper bound loses with its logit.
+template <int J, bool COH = false, bool SCORE = false, bool LAZY = false>
 __device__ __forceinline__ void topk_wave(const float* __restrict__ lrow, int E, const float* __restrict__ bias,
                                           int topk, float scale, int renorm, float* sco, int32_t* __restrict__ ids_row,
-                                          float* __restrict__ wts_row, int* ids_sh, float* wts_sh) {
+                                          float* __restrict__ wts_row, int* ids_sh, float* wts_sh,
+                                          const uint16_t* __restrict__ xrow = nullptr,
+                                          const uint16_t* __restrict__ w = nullptr, int K = 0) {
     const int lane = threadIdx.x & 63;
+    uint32_t open = 0u;                                               // LAZY: bit j = candidate j is an upper bound
     float lv[J], bv[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) {                                     // clamped addresses: every load in bounds
         const int e = min(lane + 64 * j, E - 1);
         lv[j] = COH ? ld_coherent(lrow + e) : lrow[e];
         bv[j] = bias ? bias[e] : 0.f;
+        if (LAZY) {
+            const uint32_t word = __builtin_bit_cast(uint32_t, lv[j]);
+            if (word & 0xFFFFu) open |= 1u << j;
+            lv[j] = __builtin_bit_cast(float, word & 0xFFFF0000u);
+        }
     }
+    // LAZY: the exact key of candidate e (uniform), its score stored
+    auto resolve = [&](int e) {
+        double dot = 0.0;
+        for (int k0 = 0; k0 < K; k0 += 4096) {                       // eight chunks' loads in flight (K % 512 == 0)
+            u32x4 xv[8], wv[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const int k = min(k0 + 512 * c, K - 512) + 8 * lane;
+                xv[c] = *reinterpret_cast<const u32x4*>(xrow + k);
+                wv[c] = *reinterpret_cast<const u32x4*>(w + (size_t)e * K + k);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                double part = 0.0;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    part = __builtin_fma((double)__builtin_bit_cast(float, xv[c][i] << 16),
+                                         (double)__builtin_bit_cast(float, wv[c][i] << 16), part);
+                    part = __builtin_fma((double)__builtin_bit_cast(float, xv[c][i] & 0xFFFF0000u),
+                                         (double)__builtin_bit_cast(float, wv[c][i] & 0xFFFF0000u), part);
+                }
+                dot = k0 + 512 * c < K ? dot + part : dot;           // (chunks past K re-read its last)
+            }
+        }
+        double one[1] = {dot};
+        wave_sum_scatter<1>(one, lane);
+        const float sv = (float)(1.0 / (1.0 + exp(-(double)router_round(one[0]))));
+        if (lane == 0) sco[e] = sv;
+        return topk_key(sv + (bias ? bias[e] : 0.f));
+    };
     uint32_t key[J];
     int jo[J];                                                        // key i's candidate index j
 #pragma unroll
@@ -519,6 +774,25 @@ __device__ __forceinline__ void topk_wave(const float* __restrict__ lrow, int E,
             } else {                                                  // equal keys: the lowest id
                 e = (int)wave_min_u32(key[0] == m ? (uint32_t)(64 * jo[0] + lane) : 0xFFFFFFFFu);
             }
+            if (LAZY && ((uint32_t)__builtin_amdgcn_readlane((int)open, e & 63) >> (e >> 6)) & 1u) {   // (uniform)
+                const uint32_t nk = resolve(e);
+                if (lane == (e & 63)) {                               // its key moves down to its place in the order
+                    open &= ~(1u << (e >> 6));
+                    key[0] = nk;
+#pragma unroll
+                    for (int j = 0; j + 1 < J; ++j)
+                        if (key[j + 1] > key[j] || (key[j + 1] == key[j] && jo[j + 1] < jo[j])) {
+                            const uint32_t tk = key[j];
+                            key[j] = key[j + 1];
+                            key[j + 1] = tk;
+                            const int tj = jo[j];
+                            jo[j] = jo[j + 1];
+                            jo[j + 1] = tj;
+                        }
+                }
+                --k;
+                continue;
+            }
             if (lane == (e & 63)) {                                   // the winner's lane drops its best key
 #pragma unroll
                 for (int j = 0; j + 1 < J; ++j) {
@@ -549,6 +823,17 @@ __device__ __forceinline__ void topk_wave(const float* __restrict__ lrow, int E,
             } else {
                 e = (int)wave_min_u32(bk == m ? (uint32_t)(64 * bj + lane) : 0xFFFFFFFFu);
             }
+            if (LAZY && ((uint32_t)__builtin_amdgcn_readlane((int)open, e & 63) >> (e >> 6)) & 1u) {   // (uniform)
+                const uint32_t nk = resolve(e);
+                if (lane == (e & 63)) {
+                    open &= ~(1u << (e >> 6));
+#pragma unroll
+                    for (int j = 0; j < J; ++j)
+                        if (j == (e >> 6)) key[j] = nk;
+                }
+                --k;
+                continue;
+            }
 #pragma unroll
             for (int j = 0; j < J; ++j)
                 if (j == (e >> 6) && lane == (e & 63)) key[j] = 0u;
@@ -570,20 +855,25 @@ __device__ __forceinline__ void topk_wave(const float* __restrict__ lrow, int E,
     }
 }
 
-// One wave per token, four tokens per 256-thread workgroup: topk_wave over the token's logits (scores in LDS).
-template <int J>
+// One wave per token, four tokens per 256-thread workgroup: topk_wave over the token's logits (scores in LDS), or with
+// LAZY over router_bound_kernel's words of them and the operands they bound.
+template <int J, bool LAZY = false>
 __global__ __launch_bounds__(256) void router_topk_kernel(const float* __restrict__ logits, int T, int E,
                                                           const float* __restrict__ bias, int topk, float scale,
                                                           int renorm, int32_t* __restrict__ ids,
-                                                          float* __restrict__ wts) {
+                                                          float* __restrict__ wts,
+                                                          const uint16_t* __restrict__ x = nullptr,
+                                                          int64_t x_stride = 0,
+                                                          const uint16_t* __restrict__ w = nullptr, int K = 0) {
     __shared__ float sco[4 * 64 * J];
     __shared__ int ids_sh[4 * TOPK_MAX_K];
     __shared__ float wts_sh[4 * TOPK_MAX_K];
     const int wv = threadIdx.x >> 6;
     const int t = blockIdx.x * 4 + wv;
     if (t >= T) return;                                              // uniform over the wave (no block barrier)
-    topk_wave<J>(logits + (size_t)t * E, E, bias, topk, scale, renorm, sco + wv * 64 * J, ids + (size_t)t * topk,
-                 wts + (size_t)t * topk, ids_sh + wv * TOPK_MAX_K, wts_sh + wv * TOPK_MAX_K);
+    topk_wave<J, false, false, LAZY>(logits + (size_t)t * E, E, bias, topk, scale, renorm, sco + wv * 64 * J,
+                                     ids + (size_t)t * topk, wts + (size_t)t * topk, ids_sh + wv * TOPK_MAX_K,
+                                     wts_sh + wv * TOPK_MAX_K, LAZY ? x + (size_t)t * x_stride : nullptr, w, K);
 }
 
 // The decode-size front end in one workgroup (P = T topk <= ROUTE_SMALL_MAX_P): wave w of the workgroup's nw takes
@@ -1047,8 +1337,35 @@ int launch_router_topk(const float* logits, int T, int E, const float* bias, int
     if (E > TOPK_MAX_E || topk > TOPK_MAX_K) return -1;
     const dim3 g((T + 3) / 4);
     if (T <= 0) return 0;
-    if (E <= 320) hipLaunchKernelGGL(router_topk_kernel<5>, g, dim3(256), 0, st, logits, T, E, bias, topk, scale, renorm, ids, wts);
-    else hipLaunchKernelGGL(router_topk_kernel<16>, g, dim3(256), 0, st, logits, T, E, bias, topk, scale, renorm, ids, wts);
+    if (E <= 320) hipLaunchKernelGGL(router_topk_kernel<5>, g, dim3(256), 0, st, logits, T, E, bias, topk, scale, renorm, ids, wts, nullptr, 0, nullptr, 0);
+    else hipLaunchKernelGGL(router_topk_kernel<16>, g, dim3(256), 0, st, logits, T, E, bias, topk, scale, renorm, ids, wts, nullptr, 0, nullptr, 0);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int launch_router_picks(const uint16_t* x, int64_t x_stride, const uint16_t* w, int T, int K, int E, float* bounds,
+                        const float* bias, int topk, float scale, int renorm, int32_t* ids, float* wts,
+                        hipStream_t st) {
+    if (E > TOPK_MAX_E || topk > TOPK_MAX_K || K % 512 || T <= 0) return -1;
+    if (T >= RB_BIG_T) {
+        const dim3 g((unsigned)(((T + RBB_TOK - 1) / RBB_TOK) * ((E + RBB_EXP - 1) / RBB_EXP)));
+        hipLaunchKernelGGL(router_bound_big_kernel, g, dim3(256), 0, st, x, x_stride, w, T, K, E, bounds);
+    } else {
+        const dim3 g((unsigned)(((T + 15) / 16) * ((E + 15) / 16)));
+        const int steps = K / (64 * RB_WAVES);
+        if (steps % 8 == 0)
+            hipLaunchKernelGGL(router_bound_kernel<8>, g, dim3(64 * RB_WAVES), 0, st, x, x_stride, w, T, K, E, bounds);
+        else if (steps % 4 == 0)
+            hipLaunchKernelGGL(router_bound_kernel<4>, g, dim3(64 * RB_WAVES), 0, st, x, x_stride, w, T, K, E, bounds);
+        else
+            hipLaunchKernelGGL(router_bound_kernel<1>, g, dim3(64 * RB_WAVES), 0, st, x, x_stride, w, T, K, E, bounds);
+    }
+    const dim3 g((T + 3) / 4);
+    if (E <= 320)
+        hipLaunchKernelGGL((router_topk_kernel<5, true>), g, dim3(256), 0, st, bounds, T, E, bias, topk, scale, renorm,
+                           ids, wts, x, x_stride, w, K);
+    else
+        hipLaunchKernelGGL((router_topk_kernel<16, true>), g, dim3(256), 0, st, bounds, T, E, bias, topk, scale, renorm,
+                           ids, wts, x, x_stride, w, K);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
