@@ -77,12 +77,16 @@ DecodePlan plan_decode(int64_t P, int64_t rows_bound, int64_t n, int64_t K, int6
     d.seg = d.rmax;
     d.S_cap = (int)(std::min(P, n) + (P + d.seg - 1) / d.seg);
     const int64_t s_est = std::max<int64_t>(1, std::min(P, n));
-    // K splits: the fewest that keep the staged input rows within DECODE_LDS_MAX and still give ~target 512-thread
-    // workgroups (one split needs no cross-workgroup reduction); each half of a split spans a multiple of 128
-    const int64_t target = 400;
+    // Splits of the reduction: the fewest that give more workgroups than half the CUs, whose staged input rows fit
+    // DECODE_LDS_MAX in some number of passes. One split needs no cross-workgroup reduction, and a second workgroup on
+    // a CU gains little (one already keeps its VALU nearly busy), so filling both slots of every CU (a target of 400)
+    // loses more to the partial sums than it gains. Layer call at 288 experts, hidden 4096, target 129 against 400 (and
+    // 257): intermediate 1024 T = 1 38.0 / 43.6 (42) us, 2 46.3 / 53.0 (50), 3 59.8 / 77.8 (64); intermediate 512
+    // T = 1 35.1 / 41.6, 3 42.9 / 58.7; intermediate 256 T = 3 34.3 / 49.5, 6 44.2 / 58.4 (47), 12 64.2 / 69.0.
+    const int64_t target = 129;
     int64_t sk = 0;
     for (int64_t c : {1, 2, 4, 8, 16}) {
-        if (K % c || (K / c) % 256 || decode_lds_gateup(d.rmax, (int)(K / c), shared_suh) > DECODE_LDS_MAX) continue;
+        if (K % c || (K / c) % 256 || !decode_lds_gateup(d.rmax, (int)(K / c), shared_suh)) continue;
         sk = c;
         if (s_est * (N / 128) * c >= target) break;
     }

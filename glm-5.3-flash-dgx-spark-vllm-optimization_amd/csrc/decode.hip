@@ -254,10 +254,10 @@ __device__ __forceinline__ void prio_for_quarter(int q) {
     else if (q == 2) __builtin_amdgcn_s_setprio(1);
     else __builtin_amdgcn_s_setprio(0);
 }
-// The end of quarter q of a loop of `steps` steps taken DEPTH at a time.
+// The end of part q of n of a loop of `steps` steps taken DEPTH at a time.
 template <int DEPTH>
-__device__ __forceinline__ int quarter_end(int q, int steps) {
-    return q == 3 ? steps : ((q + 1) * steps / 4) / DEPTH * DEPTH;
+__device__ __forceinline__ int part_end(int q, int n, int steps) {
+    return q == n - 1 ? steps : ((q + 1) * steps / n) / DEPTH * DEPTH;
 }
 
 // Streamed weight load: a global-address-space 16-byte load marked non-temporal (read once per call).
@@ -292,11 +292,23 @@ __device__ __forceinline__ bool arrive_fragment(unsigned long long* c, unsigned 
     return *flag != 0;
 }
 
+// LDS bytes of rn staged rows of kr reduction elements, and the passes a gate/up workgroup stages a K range of kr in: the
+// fewest of 1, 2, 4, ... whose rows fit `lds` (each pass a multiple of 256 k, so that a wave's half is whole steps).
+__host__ __device__ inline int gateup_staged(int rn, int kr, bool shared) {
+    if (shared && rn <= DUP_ROWS) return rn * (kr + 4) * 4;
+    return (shared ? 1 : 2) * rn * (kr + XPAD) * 2;
+}
+__host__ __device__ inline int gateup_passes(int rn, int kr, bool shared, int lds) {
+    int np = 1;
+    while (gateup_staged(rn, kr / np, shared) > lds && kr % (512 * np) == 0) np *= 2;
+    return np;
+}
+
 // 512 threads: workgroup = 128 gate and up columns of one segment over one K range [kc0, kc1) in chunks of kch_gu;
 // wave (cg, kh) = columns 32cg..32cg+31 over half kh of the range, DEPTH steps of loads in flight. The halves are
 // added in LDS; a fragment covering all of K runs the epilogue directly, otherwise it stores its partial in slot
 // `slot` and the fragment that completes the tile adds the slots in order. smem: the dynamic LDS.
-template <int DEPTH, bool SHARED>
+template <int DEPTH, bool SHARED, bool MULTI>
 __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, int kc0, int kc1, int slot,
                                             unsigned char* smem) {
     __shared__ int last_flag;
@@ -307,42 +319,49 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int cg = wv & 3, kh = wv >> 2;
     const int K = a.K, N = a.N, NT = N >> 4;
-    const int KR = (kc1 - kc0) * a.kch_gu, KH = KR >> 1, kbase = kc0 * a.kch_gu, RSH = KR + XPAD;
+    const int KR = (kc1 - kc0) * a.kch_gu, kbase = kc0 * a.kch_gu;
     const int KC = K / a.kch_gu;
     constexpr int NMAT = SHARED ? 1 : 2;
+    // the range is staged whole when the segment's rows fit the LDS, else in np equal passes (the accumulators stay;
+    // against a K split of such segments over two workgroups: T = 12 156 / 159 us, 64 419 / 428, 333 605 / 612)
+    const int np = MULTI ? gateup_passes(rn, KR, SHARED, a.lds_gu) : 1;
+    const int KP = KR / np, KH = KP >> 1, RSH = KP + XPAD;
     uint16_t* xs = reinterpret_cast<uint16_t*>(smem);              // [NMAT][rn][RSH] halves, or
     uint32_t* xw = reinterpret_cast<uint32_t*>(smem);              // [rn][RSD] duplicated (SHARED, rn <= DUP_ROWS)
-    const int RSD = KR + 4;
-    const bool dup = SHARED && rn <= DUP_ROWS;
+    const int RSD = KP + 4;
+    const bool dup = SHARED && rn <= DUP_ROWS && np == 1;
 
-    // prologue: the segment's rotated inputs for this K range as (row, matrix, 128-block) tasks, four per wave at
+    // prologue: the segment's rotated inputs for this pass of the K range as (row, matrix, 128-block) tasks, four per wave at
     // a time (one per 16-lane row), one quad per wave per batch. The first batch's loads are issued unconditionally
     // (task index clamped) before the weight prefetch: loads return in issue order, so inputs queued behind the
     // prefetch would wait for all of it. The segment's token ids are read once, one per lane.
-    const int g4 = lane >> 4, l16 = lane & 15;
-    const int nb = KR >> 7, ntask = rn * NMAT * nb;
+    const int g4 = lane >> 4;
+    const int nb = KP >> 7, ntask = rn * NMAT * nb;
     const int tokl = a.tok[row0 + min(lane, rn - 1)];
     const _Float16* suhg = reinterpret_cast<const _Float16*>(a.wt.g_suh[e]) + kbase;
     const _Float16* suhu = reinterpret_cast<const _Float16*>(a.wt.u_suh[e]) + kbase;
+    int pk = 0;                                                      // the pass's first k within the range
     auto task_of = [&](int c, int t0) { return t0 + 4 * (c * GU_WAVES + wv) + g4; };   // t0: batch base
-    auto task_load = [&](int task) {
+    auto stage_load = [&](int task, int toks, int ln) {             // toks: the segment's token ids, one per lane
         task = min(task, ntask - 1);
         const int r = task / (NMAT * nb), rem = task - r * NMAT * nb, mat = rem / nb, b = rem - mat * nb;
-        const int tk = __shfl(tokl, r, 64);
-        return rot8_load(a.x, (size_t)tk * a.x_stride + kbase + b * 128 + 8 * l16,
-                         (mat ? suhu : suhg) + b * 128 + 8 * l16);
+        const int tk = __shfl(toks, r, 64);
+        return rot8_load(a.x, (size_t)tk * a.x_stride + kbase + pk + b * 128 + 8 * (ln & 15),
+                         (mat ? suhu : suhg) + pk + b * 128 + 8 * (ln & 15));
     };
-    auto task_store = [&](int task, const RotIn8& vv) {
+    auto stage_store = [&](int task, const RotIn8& vv, int ln) {
         float p[8];
         rot8_scale(vv, a.xdt, p);
-        fwht128_x16s(p, lane);
-        const float hr = HAD_R * fwht_sign(lane);                    // r and the sign fwht128_x16s leaves
+        fwht128_x16s(p, ln);
+        const float hr = HAD_R * fwht_sign(ln);                      // r and the sign fwht128_x16s leaves
         const int r = task / (NMAT * nb), rem = task - r * NMAT * nb, mat = rem / nb, b = rem - mat * nb;
         if (task < ntask) {
-            if (dup) stage8_store_dup(p, hr, xw + (size_t)r * RSD, b * 128 + 8 * l16);
-            else stage8_store(p, hr, xs + (size_t)(mat * rn + r) * RSH, b * 128 + 8 * l16);
+            if (dup) stage8_store_dup(p, hr, xw + (size_t)r * RSD, b * 128 + 8 * (ln & 15));
+            else stage8_store(p, hr, xs + (size_t)(mat * rn + r) * RSH, b * 128 + 8 * (ln & 15));
         }
     };
+    auto task_load = [&](int task) { return stage_load(task, tokl, lane); };
+    auto task_store = [&](int task, const RotIn8& vv) { stage_store(task, vv, lane); };
     constexpr int QB = 1;                                            // quads per wave per batch
     constexpr int BT = 4 * QB * GU_WAVES;                            // tasks per batch
     RotIn8 v[QB];
@@ -356,9 +375,9 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
     const u32x4* U = reinterpret_cast<const u32x4*>(a.wt.u_tr[e]);
     const size_t sstr = (size_t)NT * 8 * 4;                         // one step = four k tiles
     const size_t idx0 = ((size_t)(((kbase + kh * KH) >> 4) + (t >> 1)) * NT + ct) * 8 + q;
-    const int steps = KH >> 6;                                       // a multiple of DEPTH
-    // buffer j is refilled right after use with step st + DEPTH + j; refills past the last step re-read the last
-    // step, so every load is unconditional and in bounds
+    const int steps = KH >> 6;                                       // of a pass; a multiple of DEPTH
+    // buffer j is refilled right after use with step st + DEPTH + j: the next pass's first steps past the end of a
+    // pass; refills past the last pass's end re-read its last step, so every load is unconditional and in bounds
     u32x4 gb[DEPTH], ub[DEPTH];
 #pragma unroll
     for (int j = 0; j < DEPTH; ++j) {
@@ -391,7 +410,7 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
         for (int i = 0; i < 4; ++i) xa[i] = reinterpret_cast<const u32x4*>(xr)[i];
         for (int q = 0, st = 0; q < 4; ++q) {
           prio_for_quarter(q);
-          for (const int st1 = quarter_end<DEPTH>(q, steps); st < st1; st += DEPTH) {
+          for (const int st1 = part_end<DEPTH>(q, 4, steps); st < st1; st += DEPTH) {
 #pragma unroll
             for (int j = 0; j < DEPTH; ++j) {
                 const size_t nx = idx0 + (size_t)min(st + DEPTH + j, steps - 1) * sstr;
@@ -414,6 +433,10 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
     } else {
         const uint16_t* xg = xs + (size_t)arow * RSH + kh * KH + (t >> 1) * 16;
         const uint16_t* xu = xs + (size_t)((NMAT - 1) * rn + arow) * RSH + kh * KH + (t >> 1) * 16;
+        const int qpp = max(1, 4 / np);                              // quarters of the range per pass
+        for (int pass = 0;; ++pass) {
+        const bool last_pass = !MULTI || pass + 1 == np;
+        const size_t idxp = idx0 + (size_t)pass * 2 * steps * sstr;
         u32x4 xc[2][2], xn[2][2];
         xc[0][0] = reinterpret_cast<const u32x4*>(xg)[0];
         xc[0][1] = reinterpret_cast<const u32x4*>(xg)[1];
@@ -421,12 +444,13 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
             xc[1][0] = reinterpret_cast<const u32x4*>(xu)[0];
             xc[1][1] = reinterpret_cast<const u32x4*>(xu)[1];
         }
-        for (int q = 0, st = 0; q < 4; ++q) {
-          prio_for_quarter(q);
-          for (const int st1 = quarter_end<DEPTH>(q, steps); st < st1; st += DEPTH) {
+        for (int q = 0, st = 0; q < qpp; ++q) {
+          prio_for_quarter(pass * 4 / np + q);
+          for (const int st1 = part_end<DEPTH>(q, qpp, steps); st < st1; st += DEPTH) {
 #pragma unroll
             for (int j = 0; j < DEPTH; ++j) {
-                const size_t nx = idx0 + (size_t)min(st + DEPTH + j, steps - 1) * sstr;
+                const int ns = st + DEPTH + j;
+                const size_t nx = idxp + (size_t)(ns < steps ? ns : last_pass ? steps - 1 : ns + steps) * sstr;
                 const int sn = min(st + j + 1, steps - 1);
                 const int jn = (j + 1) % DEPTH;
                 const uint32_t pgn = prev_word(gb[jn][3], lane), pun = prev_word(ub[jn][3], lane);
@@ -453,6 +477,17 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
                 pu = pun;
             }
           }
+        }
+        if (last_pass) break;
+        // the next pass's inputs; its first weights are in the buffers already
+        pk += KP;
+        __syncthreads();                                             // the staged inputs are no longer read
+        const int ln = opaque_lane(), tkl = a.tok[row0 + min(ln, rn - 1)];   // (nothing kept live across the loop)
+        for (int t0 = 0; t0 < ntask; t0 += 4 * GU_WAVES) {
+            const int task = t0 + 4 * wv + (ln >> 4);
+            stage_store(task, stage_load(task, tkl, ln), ln);
+        }
+        __syncthreads();
         }
     }
 
@@ -564,12 +599,12 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
     if (part && tid == 0) *cnt = 0ull;
 }
 
-template <int DEPTH, bool SHARED>
+template <int DEPTH, bool SHARED, bool MULTI>
 __global__ __launch_bounds__(GU_WAVES * 64) __attribute__((amdgpu_waves_per_eu(4))) void dec_gateup_kernel(
     DecodeArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     // grid (N/128, K splits, segments): split ks is chunk ks (kch_gu = K / splits), its partials in slot ks
-    gateup_tile<DEPTH, SHARED>(a, blockIdx.x, blockIdx.z, blockIdx.y, blockIdx.y + 1, blockIdx.y, smem);
+    gateup_tile<DEPTH, SHARED, MULTI>(a, blockIdx.x, blockIdx.z, blockIdx.y, blockIdx.y + 1, blockIdx.y, smem);
 }
 
 // grid (K/512, N splits, segments), 512 threads: workgroup = 512 output columns of one segment over one N range;
@@ -655,7 +690,7 @@ __device__ __forceinline__ void down_tile(const DecodeArgs& a, int cb, int s, in
     uint32_t pg = prev_word(gb[0][3], lane), pu = prev_word(ub[0][3], lane);
     for (int q = 0, st = 0; live && q < 4; ++q) {
       prio_for_quarter(q);
-      for (const int st1 = quarter_end<DEPTH>(q, steps); st < st1; st += DEPTH) {
+      for (const int st1 = part_end<DEPTH>(q, 4, steps); st < st1; st += DEPTH) {
 #pragma unroll
         for (int j = 0; j < DEPTH; ++j) {
             const size_t nx = idx0 + (size_t)min(st + DEPTH + j, steps - 1) * sstr;
@@ -852,10 +887,20 @@ int launch_rot_in(const void* x, int xdt, int64_t x_stride, const int* tok, cons
 }
 
 size_t decode_lds_gateup(int rmax, int kr, int shared_suh) {
-    size_t staged = (size_t)(shared_suh ? 1 : 2) * rmax * (kr + XPAD) * 2;
-    if (shared_suh) staged = std::max(staged, (size_t)std::min(rmax, DUP_ROWS) * (kr + 4) * 4);
+    // the largest staging of any segment of up to rmax rows that fits DECODE_LDS_MAX (0: some segment fits no pass)
+    int staged = 0;
+    for (int rn = 1; rn <= rmax; ++rn) {
+        const int b = gateup_staged(rn, kr / gateup_passes(rn, kr, shared_suh != 0, (int)DECODE_LDS_MAX), shared_suh != 0);
+        if (b > (int)DECODE_LDS_MAX) return 0;
+        staged = std::max(staged, b);
+    }
     const size_t reduce = (size_t)(4 * 64 * 16 + 2 * ZS_ROWS * 128) * 4;
-    return std::max(staged, reduce);
+    return std::max((size_t)staged, reduce);
+}
+int decode_gateup_depth(int rmax, int kr, int shared_suh) {
+    for (int rn = 1; rn <= rmax; ++rn)
+        if (kr / gateup_passes(rn, kr, shared_suh != 0, (int)DECODE_LDS_MAX) % 512) return 2;
+    return 4;
 }
 size_t decode_lds_down(int rmax, int kr) {
     return std::max((size_t)rmax * (kr + 4) * 4, (size_t)ZS_ROWS * DN_COLS * 4);
@@ -871,8 +916,10 @@ static int allow_lds(F* f) {
 static int decode_setup() {
     static bool done = false;
     if (done) return 0;
-    if (allow_lds(dec_gateup_kernel<4, true>) || allow_lds(dec_gateup_kernel<2, true>) ||
-        allow_lds(dec_gateup_kernel<4, false>) || allow_lds(dec_gateup_kernel<2, false>) ||
+    if (allow_lds(dec_gateup_kernel<4, true, false>) || allow_lds(dec_gateup_kernel<2, true, false>) ||
+        allow_lds(dec_gateup_kernel<4, false, false>) || allow_lds(dec_gateup_kernel<2, false, false>) ||
+        allow_lds(dec_gateup_kernel<4, true, true>) || allow_lds(dec_gateup_kernel<2, true, true>) ||
+        allow_lds(dec_gateup_kernel<4, false, true>) || allow_lds(dec_gateup_kernel<2, false, true>) ||
         allow_lds(dec_down_kernel<4>) || allow_lds(dec_down_kernel<2>))
         return -1;
     done = true;
@@ -884,17 +931,21 @@ int launch_decode(const DecodeArgs& a0, int rmax, hipStream_t st, int kernels) {
     if (decode_setup()) return -1;
     DecodeArgs a = a0;
     a.rmax = rmax;
-    // load depth: four steps (of 64 k) when each wave's range holds a multiple of four, else two
+    // load depth: four steps (of 64 k) when each wave's share of a pass holds a multiple of four, else two
     if (kernels & 1) {
         const dim3 grid(a.N / 128, a.sk_gu, a.S_cap);
         const size_t lds = decode_lds_gateup(rmax, a.kch_gu, a.shared_suh);
-        const bool d4 = ((a.kch_gu / 2) >> 6) % 4 == 0;
+        if (lds == 0) return 1;
+        a.lds_gu = (int)DECODE_LDS_MAX;                              // the passes are planned for it; lds covers them
+        const bool d4 = decode_gateup_depth(rmax, a.kch_gu, a.shared_suh) == 4;
+        const bool multi = gateup_passes(rmax, a.kch_gu, a.shared_suh != 0, a.lds_gu) > 1;
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(GU_WAVES * 64), lds, st, a); };
         if (a.shared_suh) {
-            if (d4) hipLaunchKernelGGL((dec_gateup_kernel<4, true>), grid, dim3(GU_WAVES * 64), lds, st, a);
-            else hipLaunchKernelGGL((dec_gateup_kernel<2, true>), grid, dim3(GU_WAVES * 64), lds, st, a);
+            if (multi) d4 ? go(dec_gateup_kernel<4, true, true>) : go(dec_gateup_kernel<2, true, true>);
+            else d4 ? go(dec_gateup_kernel<4, true, false>) : go(dec_gateup_kernel<2, true, false>);
         } else {
-            if (d4) hipLaunchKernelGGL((dec_gateup_kernel<4, false>), grid, dim3(GU_WAVES * 64), lds, st, a);
-            else hipLaunchKernelGGL((dec_gateup_kernel<2, false>), grid, dim3(GU_WAVES * 64), lds, st, a);
+            if (multi) d4 ? go(dec_gateup_kernel<4, false, true>) : go(dec_gateup_kernel<2, false, true>);
+            else d4 ? go(dec_gateup_kernel<4, false, false>) : go(dec_gateup_kernel<2, false, false>);
         }
     }
     if (kernels & 2) {

@@ -78,6 +78,7 @@ struct DecodeArgs {
     int kch_gu, kch_dn;     // chunk length (K elements for gate/up, N elements for down)
     int rmax;               // rows per segment (<= 16)
     int shared_suh;         // gate and up share one input rotation (one staged copy)
+    int lds_gu;             // LDS bytes the gate/up passes are planned for (set by launch_decode)
     float limit;
     // workspace
     float* zg;              // [K / kch_gu][2][P][N] partial sums, slot = the fragment's first chunk

@@ -1,0 +1,36 @@
+"""GPU: segments of every height around the gate/up kernel's staging limits (rows that fit the LDS in one pass, in two,
+in four; one or two staged matrices; duplicated rows), against the oracle at the kernel's rounding points (fp32 sums in
+another order: rel_l2 <= 5e-4, as for the other decode cases)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe, routing
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30))
+
+
+@pytest.mark.parametrize("K,N,shared", [(4096, 256, True), (4096, 128, False), (8192, 128, True), (6144, 128, True),
+                                        (1024, 384, False)])
+@pytest.mark.parametrize("rows", [1, 4, 5, 8, 9, 15, 16, 17, 35])
+def test_rows_per_segment(cuda, K, N, shared, rows):
+    from mi355moe import _lib, ops, synthetic
+    print(f"decode rows={rows} K={K} N={N} shared={shared}", flush=True)
+    n, topk = 5, 2
+    ex = synthetic.calibrated_layer(n, K, N, seed=11, device=cuda, shared_suh=shared)
+    x = synthetic.activations(rows, K, seed=12, device=cuda)
+    ids = torch.stack([torch.zeros(rows, dtype=torch.int32), 1 + torch.arange(rows, dtype=torch.int32) % 4], 1).to(cuda)
+    w = synthetic.softmax_weights(rows, topk, seed=13, device=cuda)
+    got = ops.moe_forward_ids(ex, x, ids, w, out_dtype=torch.float32, path=_lib.PATH_DECODE).cpu().numpy()
+    lay = {k: getattr(ex, k).cpu().numpy() for k in ("w13_trellis", "w13_suh", "w13_svh", "w2_trellis", "w2_suh",
+                                                     "w2_svh")}
+    tok, e, w16 = moe.pairs_from_routing(routing.map_topk_to_local(ids.cpu().numpy(), n, None), w.cpu().numpy(), n, topk)
+    ref = moe.forward(lay, x.cpu().to(torch.float16).numpy(), tok, e, w16, 10.0, "decode_x")
+    assert np.isfinite(got).all()
+    assert _rel(got, ref) <= 5e-4
