@@ -53,6 +53,11 @@ int tok_rows_flag(const mi355moe_exl3_layer* L) {
     return (L->flags & MI355MOE_LAYER_SHARED_W13_SUH) && (L->flags & MI355MOE_LAYER_UNIFORM_W13_SUH) ? 1 : 0;
 }
 
+// Pairs of P expected on n local experts: with an expert map over more global ids, their share of the ids.
+int64_t local_pairs(int64_t P, int64_t n, const int64_t* expert_map, int64_t n_global) {
+    return expert_map && n_global > n ? std::max<int64_t>(1, P * n / n_global) : P;
+}
+
 // The one-launch schedule's lag in segments of one ticket queue (pf_sched_item): MI355MOE_SCHED_LAG, default 0 = all
 // of a queue's gate/up items before its first down item (a down item then rarely waits; small lags make down items
 // wait for gate/up items still running).
@@ -614,6 +619,7 @@ static int run_grouped(const mi355moe_exl3_layer* layer, const void* x, int x_dt
     d.out_stride = out_stride;
     d.e4m3 = e4m3 ? 1 : 0;
     d.tok_rows = tok_rows_flag(layer);
+    d.pairs_local = (int)local_pairs(P, n, expert_map, n_global);
     d.contrib_bf16 = (options & MI355MOE_OPT_BF16_CONTRIB) ? 1 : 0;
     d.out_accumulate = (options & MI355MOE_OPT_ACCUMULATE) ? 1 : 0;
     if ((stages & MI355MOE_STAGE_GATEUP) && (stages & MI355MOE_STAGE_DOWN)) {
@@ -867,6 +873,7 @@ int mi355moe_moe_forward_ids_split(const mi355moe_exl3_layer* layer, const void*
     a.x_stride = x_stride;
     a.tok = w.fat.tok;
     a.tok_rows = tok_rows_flag(layer);
+    a.pairs_local = (int)local_pairs(P, n, expert_map, n_global);
     a.w16 = w.fat.w16;
     a.pe = w.fat.pe;
     a.inv = w.fat.inv;

@@ -161,6 +161,7 @@ struct PrefillArgs {
     int* sched;
     int sched_lag;
     int sched_force;
+    int pairs_local;        // pairs expected on this rank's experts (the tile choice); 0: P
 };
 constexpr int PREFILL_TM = 256;
 constexpr int PF_SCHED_QUEUES = 8;      // ticket queues (one per XCD; segment s in queue s % 8)

@@ -1607,7 +1607,9 @@ int prefill_setup() {
 //   T = 4096 (~114 rows):            mid 29 % faster / mid 21 % faster (small 3 % slower);
 //   T = 6144 (~171 rows):            mid 4 % slower;
 //   T = 8192 (~228 rows):            mid 8 % slower, small 47 % slower; Zipf-skewed routing: mid 4 % faster.
-// Hence: P <= 64 n: mid (small for e4m3); P <= 128 n: mid; larger calls: the 256-row kernels. "hybrid" splits a
+// Hence: P <= 64 n: mid (small for e4m3); P <= 128 n: mid; larger calls: the 256-row kernels. P is the pairs
+// expected on this call's experts: with an expert map only the share n / n_global of the routed ones (144 of 288
+// experts, T = 4289, Zipf routing, 119 rows per expert: mid 823 us, 256-row tiles 931). "hybrid" splits a
 // call by segment size (segments of at most PF_SMALL_ROWS rows on the small tiles, larger ones on the 256-row
 // tiles). The environment variable MI355MOE_PREFILL_TILES = "small", "mid", "large" or "hybrid" forces a choice;
 // all give bit-identical results (a row's arithmetic does not depend on the tile that holds it).
@@ -1620,7 +1622,7 @@ static int pf_tiles(const PrefillArgs& a) {
     if (f && !strcmp(f, "large")) return PF_TILES_LARGE;
     if (f && !strcmp(f, "hybrid")) return PF_TILES_BOTH;
     if (a.n <= 0) return PF_TILES_LARGE;
-    const int64_t P = a.P, n = a.n;
+    const int64_t P = a.pairs_local > 0 ? a.pairs_local : a.P, n = a.n;
     if (P <= 64 * n) return a.e4m3 ? PF_TILES_SMALL : PF_TILES_MID;
     return P <= 128 * n ? PF_TILES_MID : PF_TILES_LARGE;
 }
