@@ -1,0 +1,38 @@
+"""GPU: one expert-parallel rank of a layer on the grouped tier. Its tile kind follows the pairs expected on its own
+experts, and the combine skips the slots of other ranks; both are bit-identical to the 256-row tiles over the same
+routing, and the output matches the oracle (rel_l2 <= 5e-4, the bar of the other grouped cases)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe, routing
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,topk,local", [(300, 4, 8), (300, 4, 1), (257, 9, 4), (130, 1, 2)])
+def test_rank(cuda, monkeypatch, T, topk, local):
+    from mi355moe import _lib, ops, synthetic
+    n_global, K, N = 16, 512, 256
+    print(f"ep rank T={T} topk={topk} local={local} of {n_global}", flush=True)
+    ex = synthetic.calibrated_layer(local, K, N, seed=21, device=cuda, uniform_suh=True)
+    x = synthetic.activations(T, K, seed=22, device=cuda)
+    g = torch.Generator().manual_seed(23)
+    ids = torch.rand(T, n_global, generator=g).topk(topk, 1).indices.to(torch.int32).to(cuda)
+    w = synthetic.softmax_weights(T, topk, seed=24, device=cuda)
+    emap = torch.full((n_global,), -1, dtype=torch.int64)
+    emap[3:3 + local] = torch.arange(local)                          # tokens without a local expert among them
+    got = {}
+    for tiles in ("auto", "large"):
+        monkeypatch.setenv("MI355MOE_PREFILL_TILES", tiles)
+        got[tiles] = ops.moe_forward_ids(ex, x, ids, w, out_dtype=torch.float32, expert_map=emap.to(cuda),
+                                         path=_lib.PATH_PREFILL).cpu().numpy()
+    assert np.array_equal(got["auto"], got["large"])
+    lay = {k: getattr(ex, k).cpu().numpy() for k in ("w13_trellis", "w13_suh", "w13_svh", "w2_trellis", "w2_suh",
+                                                     "w2_svh")}
+    tok, e, w16 = moe.pairs_from_routing(routing.map_topk_to_local(ids.cpu().numpy(), local, emap.numpy()),
+                                         w.cpu().numpy(), local, topk)
+    ref = moe.forward(lay, x.cpu().to(torch.float16).numpy(), tok, e, w16, 10.0, "e3")
+    assert np.linalg.norm(got["auto"] - ref) <= 5e-4 * np.linalg.norm(ref)
