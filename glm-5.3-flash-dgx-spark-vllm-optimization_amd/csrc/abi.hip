@@ -66,6 +66,14 @@ int sched_lag() {
     return v ? std::max(0, atoi(v)) : 0;
 }
 
+// Whether a decode call of a layer with one w13 suh rotates its tokens' rows first, in a launch of their own: every
+// gate/up workgroup then copies its segment's staged rows instead of rotating them (each of the N / 128 column blocks
+// of each of a token's experts rotated it again: 23 % of the kernel's VALU instructions at 9 rows per expert). The
+// launch costs 4 - 6 us, which 1.5 pairs per expert pay for (288 experts, hidden 4096, intermediate 1024, rotated first
+// / in the workgroups: T = 8 118 / 115 us, 24 260 / 257, 32 303 / 304, 64 399 / 406, 128 479 / 498, 333 539 / 594,
+// 500 658 / 732).
+bool rotate_first(int64_t P, int64_t n) { return 2 * P >= 3 * n; }
+
 struct DecodePlan {
     int rmax, seg, S_cap, sk_gu, sk_dn, kch_gu, kch_dn;
 };
@@ -568,6 +576,7 @@ static int prep_decode(const mi355moe_exl3_layer* layer, const void* x, int x_dt
     d.kch_gu = p.kch_gu;
     d.kch_dn = p.kch_dn;
     d.shared_suh = shared_flag(layer);
+    if (tok_rows_flag(layer) && rotate_first(P, n)) d.xrot = reinterpret_cast<uint16_t*>(d.contrib);   // [T][K] of [P][2K]
     d.limit = limit;
     d.out = out;
     d.odt = dt_w(out_dtype);

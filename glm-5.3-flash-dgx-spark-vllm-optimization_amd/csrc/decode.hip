@@ -18,6 +18,8 @@
 //            suh_d)) * r)
 //   down     v = H(sum_n xd Wq_d) * (r * w16) * svh_d                   (exl3.cu:455-496)
 //   combine  out[t] = sum over the token's slots in slot order (exl3.cu:815-864), or fp32 atomics (accumulate mode)
+#include <cstring>
+
 #include "common.cuh"
 #include "mi355moe_internal.h"
 
@@ -308,7 +310,7 @@ __host__ __device__ inline int gateup_passes(int rn, int kr, bool shared, int ld
 // wave (cg, kh) = columns 32cg..32cg+31 over half kh of the range, DEPTH steps of loads in flight. The halves are
 // added in LDS; a fragment covering all of K runs the epilogue directly, otherwise it stores its partial in slot
 // `slot` and the fragment that completes the tile adds the slots in order. smem: the dynamic LDS.
-template <int DEPTH, bool SHARED, bool MULTI>
+template <int DEPTH, bool SHARED, bool MULTI, bool PRE>
 __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, int kc0, int kc1, int slot,
                                             unsigned char* smem) {
     __shared__ int last_flag;
@@ -365,8 +367,51 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
     constexpr int QB = 1;                                            // quads per wave per batch
     constexpr int BT = 4 * QB * GU_WAVES;                            // tasks per batch
     RotIn8 v[QB];
+    // PRE: the rows were rotated once per token (xrot, already in the staged order), so staging is a copy: LDS DMA for
+    // rows staged as halves (every wave instruction 512 k of one row), 16-byte loads for duplicated ones
+    const bool dma = PRE && !dup && (KP & 511) == 0;
+    const int cpr = KP >> 3, nchunk = rn * cpr;                      // 16-byte chunks per row, in all
+    constexpr int PB = 4;                                            // chunks per thread per batch
+    u32x4 xv[PRE ? PB : 1];
+    auto pre_dma = [&](int toks, int ln) {
+        const int ni = KP >> 9, tot = rn * ni;
+        for (int i = wv; i < tot; i += GU_WAVES) {                   // (uniform)
+            const int r = i / ni, j = i - r * ni;
+            const uint16_t* src = a.xrot + (size_t)__builtin_amdgcn_readlane(toks, r) * K + kbase + pk + 512 * j;
+            dma16(src + 8 * ln, reinterpret_cast<unsigned char*>(xs + (size_t)r * RSH + 512 * j));
+        }
+    };
+    auto pre_load = [&](int i, int toks) {
+        i = min(i, nchunk - 1);
+        const int r = i / cpr, k = 8 * (i - r * cpr);
+        return ld_g128(a.xrot + (size_t)__shfl(toks, r, 64) * K + kbase + pk + k);
+    };
+    auto pre_store = [&](int i, const u32x4& w) {
+        if (i >= nchunk) return;
+        const int r = i / cpr, k = 8 * (i - r * cpr);
+        if (dup) {
+            u32x4* d = reinterpret_cast<u32x4*>(xw + (size_t)r * RSD + k);
 #pragma unroll
-    for (int c = 0; c < QB; ++c) v[c] = task_load(task_of(c, 0));
+            for (int m = 0; m < 2; ++m) {
+                const uint32_t w0 = w[2 * m], w1 = w[2 * m + 1];
+                d[m] = u32x4{__builtin_amdgcn_perm(w0, w0, 0x01000100u), __builtin_amdgcn_perm(w0, w0, 0x03020302u),
+                             __builtin_amdgcn_perm(w1, w1, 0x01000100u), __builtin_amdgcn_perm(w1, w1, 0x03020302u)};
+            }
+        } else {
+            *reinterpret_cast<u32x4*>(xs + (size_t)r * RSH + k) = w;
+        }
+    };
+    if constexpr (PRE) {
+        if (dma) {
+            pre_dma(tokl, lane);
+        } else {
+#pragma unroll
+            for (int c = 0; c < PB; ++c) xv[c] = pre_load(tid + c * GU_WAVES * 64, tokl);
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < QB; ++c) v[c] = task_load(task_of(c, 0));
+    }
     __builtin_amdgcn_sched_barrier(0);
 
     const int t = lane >> 3, q = lane & 7;
@@ -387,13 +432,28 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
     __builtin_amdgcn_sched_barrier(0);
 
     // the first batch in straight-line code (so its wait leaves the prefetch in flight), then any further batches
+    if constexpr (PRE) {
+        if (dma) {
+            WAIT_VM(0);                                              // this wave's DMA has landed
+        } else {
 #pragma unroll
-    for (int c = 0; c < QB; ++c) task_store(task_of(c, 0), v[c]);
-    for (int t0 = BT; t0 < ntask; t0 += BT) {
+            for (int c = 0; c < PB; ++c) pre_store(tid + c * GU_WAVES * 64, xv[c]);
+            for (int i0 = tid + PB * GU_WAVES * 64; i0 - tid < nchunk; i0 += PB * GU_WAVES * 64) {
 #pragma unroll
-        for (int c = 0; c < QB; ++c) v[c] = task_load(task_of(c, t0));
+                for (int c = 0; c < PB; ++c) xv[c] = pre_load(i0 + c * GU_WAVES * 64, tokl);
 #pragma unroll
-        for (int c = 0; c < QB; ++c) task_store(task_of(c, t0), v[c]);
+                for (int c = 0; c < PB; ++c) pre_store(i0 + c * GU_WAVES * 64, xv[c]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < QB; ++c) task_store(task_of(c, 0), v[c]);
+        for (int t0 = BT; t0 < ntask; t0 += BT) {
+#pragma unroll
+            for (int c = 0; c < QB; ++c) v[c] = task_load(task_of(c, t0));
+#pragma unroll
+            for (int c = 0; c < QB; ++c) task_store(task_of(c, t0), v[c]);
+        }
     }
     __syncthreads();
 
@@ -483,9 +543,19 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
         pk += KP;
         __syncthreads();                                             // the staged inputs are no longer read
         const int ln = opaque_lane(), tkl = a.tok[row0 + min(ln, rn - 1)];   // (nothing kept live across the loop)
-        for (int t0 = 0; t0 < ntask; t0 += 4 * GU_WAVES) {
-            const int task = t0 + 4 * wv + (ln >> 4);
-            stage_store(task, stage_load(task, tkl, ln), ln);
+        if constexpr (PRE) {
+            if (dma) {
+                pre_dma(tkl, ln);
+                WAIT_VM(0);
+            } else {
+                const int td = 64 * wv + ln;
+                for (int i0 = td; i0 - td < nchunk; i0 += GU_WAVES * 64) pre_store(i0, pre_load(i0, tkl));
+            }
+        } else {
+            for (int t0 = 0; t0 < ntask; t0 += 4 * GU_WAVES) {
+                const int task = t0 + 4 * wv + (ln >> 4);
+                stage_store(task, stage_load(task, tkl, ln), ln);
+            }
         }
         __syncthreads();
         }
@@ -599,12 +669,12 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
     if (part && tid == 0) *cnt = 0ull;
 }
 
-template <int DEPTH, bool SHARED, bool MULTI>
+template <int DEPTH, bool SHARED, bool MULTI, bool PRE = false>
 __global__ __launch_bounds__(GU_WAVES * 64) __attribute__((amdgpu_waves_per_eu(4))) void dec_gateup_kernel(
     DecodeArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     // grid (N/128, K splits, segments): split ks is chunk ks (kch_gu = K / splits), its partials in slot ks
-    gateup_tile<DEPTH, SHARED, MULTI>(a, blockIdx.x, blockIdx.z, blockIdx.y, blockIdx.y + 1, blockIdx.y, smem);
+    gateup_tile<DEPTH, SHARED, MULTI, PRE>(a, blockIdx.x, blockIdx.z, blockIdx.y, blockIdx.y + 1, blockIdx.y, smem);
 }
 
 // grid (K/512, N splits, segments), 512 threads: workgroup = 512 output columns of one segment over one N range;
@@ -920,6 +990,8 @@ static int decode_setup() {
         allow_lds(dec_gateup_kernel<4, false, false>) || allow_lds(dec_gateup_kernel<2, false, false>) ||
         allow_lds(dec_gateup_kernel<4, true, true>) || allow_lds(dec_gateup_kernel<2, true, true>) ||
         allow_lds(dec_gateup_kernel<4, false, true>) || allow_lds(dec_gateup_kernel<2, false, true>) ||
+        allow_lds(dec_gateup_kernel<4, true, false, true>) || allow_lds(dec_gateup_kernel<2, true, false, true>) ||
+        allow_lds(dec_gateup_kernel<4, true, true, true>) || allow_lds(dec_gateup_kernel<2, true, true, true>) ||
         allow_lds(dec_down_kernel<4>) || allow_lds(dec_down_kernel<2>))
         return -1;
     done = true;
@@ -940,7 +1012,22 @@ int launch_decode(const DecodeArgs& a0, int rmax, hipStream_t st, int kernels) {
         const bool d4 = decode_gateup_depth(rmax, a.kch_gu, a.shared_suh) == 4;
         const bool multi = gateup_passes(rmax, a.kch_gu, a.shared_suh != 0, a.lds_gu) > 1;
         auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(GU_WAVES * 64), lds, st, a); };
-        if (a.shared_suh) {
+        if (a.shared_suh && a.xrot) {
+            PrefillArgs g;
+            memset(&g, 0, sizeof(g));
+            g.wt = a.wt;
+            g.n = a.n;
+            g.K = a.K;
+            g.T = a.T;
+            g.x = a.x;
+            g.xdt = a.xdt;
+            g.x_stride = a.x_stride;
+            g.tok_rows = 1;
+            g.h13 = a.xrot;
+            if (launch_gather_tokens(g, st)) return -1;
+            if (multi) d4 ? go(dec_gateup_kernel<4, true, true, true>) : go(dec_gateup_kernel<2, true, true, true>);
+            else d4 ? go(dec_gateup_kernel<4, true, false, true>) : go(dec_gateup_kernel<2, true, false, true>);
+        } else if (a.shared_suh) {
             if (multi) d4 ? go(dec_gateup_kernel<4, true, true>) : go(dec_gateup_kernel<2, true, true>);
             else d4 ? go(dec_gateup_kernel<4, true, false>) : go(dec_gateup_kernel<2, true, false>);
         } else {

@@ -60,6 +60,9 @@ struct DecodeArgs {
     const void* x;
     int xdt;                // DT_F16 or DT_BF16
     int64_t x_stride;       // elements
+    uint16_t* xrot;         // optional, layers whose experts share one w13 suh: [T][K] fp16, the tokens' rotated rows
+                            // in the staged order (xa_pos), written before gate/up by launch_decode (may alias
+                            // contrib, which the down kernel fills after the last read)
     // routing tables (sorted position order)
     const int* tok;
     const uint16_t* w16;
@@ -311,6 +314,7 @@ int launch_decode(const DecodeArgs& a, int rmax, hipStream_t st, int kernels = 7
 size_t decode_lds_gateup(int rmax, int kr, int shared_suh);
 size_t decode_lds_down(int rmax, int kr);
 constexpr size_t DECODE_LDS_MAX = 81920;   // two 512-thread workgroups per CU
+int launch_gather_tokens(const PrefillArgs& a, hipStream_t st);
 int launch_dequant(const uint16_t* trellis, int kt, int nt, uint16_t* wq, hipStream_t st);
 int launch_sigmoid(const float* g, int64_t n, int variant, float* out, hipStream_t st);
 int launch_rot_in(const void* x, int xdt, int64_t x_stride, const int* tok, const int* pe, const int64_t* suh_tab,

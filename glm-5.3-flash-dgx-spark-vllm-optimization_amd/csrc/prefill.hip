@@ -1633,6 +1633,12 @@ static int pf_tiles(const PrefillArgs& a) {
     return P <= 128 * n ? PF_TILES_MID : PF_TILES_LARGE;
 }
 
+// One rotated row per token (a.tok_rows) into h13.
+int launch_gather_tokens(const PrefillArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL(pf_gather_kernel, dim3(std::max(1, std::min(4096, (a.T + 3) / 4))), dim3(256), 0, st, a);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 int launch_prefill(const PrefillArgs& a0, hipStream_t st, int kernels) {
     if (prefill_setup()) return -1;
     PrefillArgs a = a0;

@@ -16,14 +16,11 @@ def _rel(a, b):
     return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30))
 
 
-@pytest.mark.parametrize("K,N,shared", [(4096, 256, True), (4096, 128, False), (8192, 128, True), (6144, 128, True),
-                                        (1024, 384, False)])
-@pytest.mark.parametrize("rows", [1, 4, 5, 8, 9, 15, 16, 17, 35])
-def test_rows_per_segment(cuda, K, N, shared, rows):
+def _check(cuda, K, N, rows, **suh):
     from mi355moe import _lib, ops, synthetic
-    print(f"decode rows={rows} K={K} N={N} shared={shared}", flush=True)
+    print(f"decode rows={rows} K={K} N={N} {suh}", flush=True)
     n, topk = 5, 2
-    ex = synthetic.calibrated_layer(n, K, N, seed=11, device=cuda, shared_suh=shared)
+    ex = synthetic.calibrated_layer(n, K, N, seed=11, device=cuda, **suh)
     x = synthetic.activations(rows, K, seed=12, device=cuda)
     ids = torch.stack([torch.zeros(rows, dtype=torch.int32), 1 + torch.arange(rows, dtype=torch.int32) % 4], 1).to(cuda)
     w = synthetic.softmax_weights(rows, topk, seed=13, device=cuda)
@@ -34,3 +31,18 @@ def test_rows_per_segment(cuda, K, N, shared, rows):
     ref = moe.forward(lay, x.cpu().to(torch.float16).numpy(), tok, e, w16, 10.0, "decode_x")
     assert np.isfinite(got).all()
     assert _rel(got, ref) <= 5e-4
+
+
+@pytest.mark.parametrize("K,N,shared", [(4096, 256, True), (4096, 128, False), (8192, 128, True), (6144, 128, True),
+                                        (1024, 384, False)])
+@pytest.mark.parametrize("rows", [1, 4, 5, 8, 9, 15, 16, 17, 35])
+def test_rows_per_segment(cuda, K, N, shared, rows):
+    _check(cuda, K, N, rows, shared_suh=shared)
+
+
+# one w13 suh for every expert: from 4 rows here (1.5 pairs per expert) the rows are rotated once per token and copied,
+# by LDS DMA where a pass is whole 512-k pieces, by register loads where it is not or where the rows are duplicated
+@pytest.mark.parametrize("K,N", [(4096, 256), (8192, 128), (6144, 128), (768, 128), (256, 128), (10240, 128)])
+@pytest.mark.parametrize("rows", [3, 4, 5, 9, 16, 17, 35])
+def test_rows_rotated_once(cuda, K, N, rows):
+    _check(cuda, K, N, rows, uniform_suh=True)
