@@ -279,6 +279,28 @@ __device__ __forceinline__ void dma16(const void* src_lane, unsigned char* lds_w
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(m0), "v"(src_lane)
                  : "memory", "m0");
 }
+// A wave-uniform address made scalar.
+template <typename T>
+__device__ __forceinline__ const T* uniform_ptr(const T* p) {
+    const uint64_t v = (uint64_t)(uintptr_t)p;
+    const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) |
+                       ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32);
+    return reinterpret_cast<const T*>((uintptr_t)u);
+}
+// The same with a wave-uniform base and a 32-bit byte offset per lane (no 64-bit address arithmetic on the VALU);
+// COH: as dma16_coh below.
+template <bool COH = false>
+__device__ __forceinline__ void dma16_base(const void* base, uint32_t off_lane, unsigned char* lds_wave) {
+    const uint32_t m0 = (uint32_t)(uintptr_t)lds_wave;
+    if constexpr (COH)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 sc1" ::"s"(m0), "v"(off_lane),
+                     "s"(base)
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0), "v"(off_lane),
+                     "s"(base)
+                     : "memory", "m0");
+}
 // The same marked non-temporal (data read once, e.g. streamed weights).
 __device__ __forceinline__ void dma16_nt(const void* src_lane, unsigned char* lds_wave) {
     const uint32_t m0 = (uint32_t)(uintptr_t)lds_wave;

@@ -546,7 +546,7 @@ __device__ __forceinline__ uint32_t pf_decode_pair(const uint32_t (&w)[3], int p
 // step it + NS - 1 are issued while step it is multiplied).
 template <bool E4M3 = false, int NRB = 8, int TM = PF_TM, int NS = PF_NS, bool ACOH = false>
 __device__ __forceinline__ void pf_gemm(const PfTile& t, unsigned char* smem, f16v (&acc)[8][2]) {
-    static_assert(32 * NRB <= TM && TM % 32 == 0, "the multiplied row blocks are staged");
+    static_assert(32 * NRB <= TM && TM % 32 == 0 && (NRB == 8 || NRB == 4 || NRB == 2), "the multiplied row blocks are staged");
     constexpr int ASB = TM * PF_RB;                                   // one A stage
     constexpr int CPR = PF_RB / 16;                                   // 16-byte chunks per A row
     constexpr int RPW = TM / 4;                                       // A rows staged by each wave
@@ -558,42 +558,32 @@ __device__ __forceinline__ void pf_gemm(const PfTile& t, unsigned char* smem, f1
     const int tid = opaque_tid(), lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int steps = t.kdim / (16 * PF_KT);
-    // A DMA sources: instruction i of this wave = rows RPW wv + RPI i + lane / CPR, slot lane % CPR
-    const uint16_t* asrc[NA];
+    // A DMA sources: instruction i of this wave = rows RPW wv + RPI i + lane / CPR, slot lane % CPR (byte offsets from
+    // a_rows: below 2^32, the host keeps token-row buffers of more bytes off this path)
+    uint32_t aoff[NA];
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
         const int R = RPW * wv + RPI * i + lane / CPR;
         const int chunk = (lane % CPR) ^ pf_swz(R);
         const int rr = min(R, t.rn - 1);
-        asrc[i] = t.a_rows + (size_t)(t.a_tok ? t.a_tok[rr] : rr) * t.kdim + 8 * chunk;
+        aoff[i] = (uint32_t)(t.a_tok ? t.a_tok[rr] : rr) * (uint32_t)(2 * t.kdim) + 16 * chunk;
     }
     // raw-word DMA sources: instruction i, lane -> k tile 2i + lane / 32, column tile (lane / 8) % 4, piece lane % 8
-    const uint32_t* wsrc = t.btr + ((size_t)(lane >> 5) * t.btiles_n + t.bcol0 + ((lane >> 3) & 3)) * 32 + 4 * (lane & 7);
-    const size_t wstep = (size_t)PF_KT * t.btiles_n * 32;             // words per step (PF_KT k tiles)
-    const size_t wins = (size_t)2 * t.btiles_n * 32;                  // words between a wave's W instructions
-    auto issue_w = [&](int sw) {
-        unsigned char* wd = Wst + (sw % NS) * PF_WSB + wv * PF_WWB;
-#pragma unroll
-        for (int i = 0; i < PF_KT / 2; ++i) dma16(wsrc + (size_t)sw * wstep + i * wins, wd + i * 1024);
-    };
-    auto issue_one = [&](int k, int sa, int sw) {                     // DMA instruction k of the batch (A(sa), W(sw))
+    const uint32_t woff = (uint32_t)((lane >> 5) * t.btiles_n + ((lane >> 3) & 3)) * 128 + 16 * (lane & 7);
+    const unsigned char* wbase = uniform_ptr(reinterpret_cast<const unsigned char*>(t.btr) + (size_t)t.bcol0 * 128);
+    const unsigned char* abase = uniform_ptr(reinterpret_cast<const unsigned char*>(t.a_rows));
+    const uint32_t wstep = (uint32_t)PF_KT * t.btiles_n * 128;        // bytes per step (PF_KT k tiles)
+    const uint32_t wins = (uint32_t)2 * t.btiles_n * 128;             // bytes between a wave's W instructions
+    // instruction k of the batch A(sa) -> stage da, W(sw) -> stage dw
+    auto issue_one = [&](int k, int sa, int da, int sw, int dw) {
         sa = min(sa, steps - 1);
         sw = min(sw, steps - 1);
-        if (k < NA && ACOH)
-            dma16_coh(asrc[k] + (size_t)sa * 16 * PF_KT, Ast + (sa % NS) * ASB + wv * RPW * PF_RB + k * 1024);
-        else if (k < NA)
-            dma16(asrc[k] + (size_t)sa * 16 * PF_KT, Ast + (sa % NS) * ASB + wv * RPW * PF_RB + k * 1024);
+        if (k < NA)
+            dma16_base<ACOH>(abase + (uint32_t)sa * (uint32_t)PF_RB, aoff[k],
+                             Ast + da * ASB + wv * RPW * PF_RB + k * 1024);
         else
-            dma16(wsrc + (size_t)sw * wstep + (k - NA) * wins, Wst + (sw % NS) * PF_WSB + wv * PF_WWB + (k - NA) * 1024);
-    };
-    auto issue = [&](int sa, int sw) {                                // the whole batch
-#pragma unroll
-        for (int k = 0; k < NDMA; ++k) issue_one(k, sa, sw);
-    };
-    auto words = [&](int sw, uint32_t (&w)[PF_KT][3]) {              // this lane's raw words of step sw
-        const unsigned char* wr = Wst + (sw % NS) * PF_WSB + wv * PF_WWB;
-#pragma unroll
-        for (int kt = 0; kt < PF_KT; ++kt) pf_load_words(wr + kt * 512, lane, w[kt]);
+            dma16_base(wbase + (size_t)sw * wstep + (k - NA) * wins, woff,
+                       Wst + dw * PF_WSB + wv * PF_WWB + (k - NA) * 1024);
     };
     auto operands = [&](uint32_t (&q)[PF_KT][8], h8 (&b)[PF_KT][2]) {   // decoded pairs -> B operands
 #pragma unroll
@@ -606,48 +596,85 @@ __device__ __forceinline__ void pf_gemm(const PfTile& t, unsigned char* smem, f1
             b[kt][1] = __builtin_bit_cast(h8, u32x4{q[kt][2], q[kt][3], q[kt][6], q[kt][7]});
         }
     };
-    auto afrag = [&](const unsigned char* as, int i) {                // A fragment i = (k tile i / 8, rows 32 (i % 8))
-        const int R = 32 * (i & 7) + (lane & 31);
-        const int slot = (2 * (i >> 3) + (lane >> 5)) ^ pf_swz(R);
-        return *reinterpret_cast<const h8*>(as + R * PF_RB + 16 * slot);
+    // This lane's LDS offsets inside a stage, kept in registers (a step adds the stage's offset, the row block and the
+    // k tile's words are immediates): A fragments of k tile kt (row lane % 32, chunk 2 kt + lane / 32, swizzled; the
+    // swizzle does not depend on the row block), raw words wp and wp - 1.
+    uint32_t la[PF_KT], lw, lp;
+    {
+        const int R = lane & 31, wp = 4 * (lane & 7) + 2 * (lane >> 5), tile = (lane & 31) >> 3;
+#pragma unroll
+        for (int kt = 0; kt < PF_KT; ++kt) la[kt] = R * PF_RB + 16 * ((2 * kt + (lane >> 5)) ^ pf_swz(R));
+        lw = NS * ASB + wv * PF_WWB + tile * 128 + 4 * wp;
+        lp = NS * ASB + wv * PF_WWB + tile * 128 + 4 * ((wp + 31) & 31);
+#pragma unroll
+        for (int kt = 0; kt < PF_KT; ++kt) asm volatile("" : "+v"(la[kt]));
+        asm volatile("" : "+v"(lw), "+v"(lp));
+    }
+    auto words = [&](int stage, uint32_t (&w)[PF_KT][3]) {           // this lane's raw words of a stage
+        const unsigned char* p2 = smem + lw + stage * PF_WSB;
+        const unsigned char* p1 = smem + lp + stage * PF_WSB;
+#pragma unroll
+        for (int kt = 0; kt < PF_KT; ++kt) {
+            const uint2 v = *reinterpret_cast<const uint2*>(p2 + kt * 512);
+            w[kt][0] = *reinterpret_cast<const uint32_t*>(p1 + kt * 512);
+            w[kt][1] = v.x;
+            w[kt][2] = v.y;
+        }
     };
-    // One step, in a fixed instruction order (one wave per SIMD issues everything itself): the 16 PF_KT MFMAs of
-    // step it, each pair with one fp16 pair's decode for step it + 1 between them (VALU work issued while the MFMAs
-    // run), the A fragments read four MFMA pairs ahead.
-    constexpr int NF = 8 * PF_KT;                                     // A fragments (and decoded pairs) per step
-    constexpr int DMA_EVERY = NF / NDMA;                              // MFMA pairs between DMA instructions
-    auto step = [&](int it, const h8 (&bc)[PF_KT][2], h8 (&bn)[PF_KT][2]) {
-        WAIT_VM(NDMA * (NS - 2));                                  // A(it) and words(it + 1): the oldest batch
+    // One step (stage st = it % NS), in a fixed instruction order (a wave issues everything itself): the 2 NRB PF_KT
+    // MFMAs of step it spread evenly over the 8 PF_KT pair decodes for step it + 1 (VALU work issued while the MFMAs
+    // run; the last step decodes nothing), the A fragments read four ahead.
+    constexpr int NF = 8 * PF_KT;                                     // decoded pairs per step
+    constexpr int NM = 2 * NRB * PF_KT;                               // MFMAs per step
+    constexpr int NFR = NRB * PF_KT;                                  // A fragments per step: k tile f / NRB, block f % NRB
+    constexpr int DMA_EVERY = NF / NDMA;                              // pairs between DMA instructions
+    auto step = [&](auto lastc, int it, int st, const h8 (&bc)[PF_KT][2], h8 (&bn)[PF_KT][2]) {
+        constexpr int LAST = decltype(lastc)::value;                  // 0; 1 or 2: the last step but one, the last one
+        constexpr int QUEUED = LAST == 2 ? NS - 3 : NS - 2;           // batches issued after the one waited for
+        WAIT_VM(NDMA * QUEUED);                                       // A(it) and words(it + 1): the oldest batch
         LDS_BARRIER();
         __builtin_amdgcn_sched_barrier(0);
-        const unsigned char* as = Ast + (it % NS) * ASB;
+        const int st1 = st + 1 == NS ? 0 : st + 1, stp = st == 0 ? NS - 1 : st - 1;
         uint32_t w[PF_KT][3];
-        words(it + 1, w);                                             // step it + 1 (past the end: never used)
-        h8 af[NF];
+        if (LAST != 2) words(st1, w);
+        const unsigned char* pa[PF_KT];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (i < NRB) af[i] = afrag(as, i);
+        for (int kt = 0; kt < PF_KT; ++kt) pa[kt] = smem + la[kt] + st * ASB;
+        auto afrag = [&](int f) { return *reinterpret_cast<const h8*>(pa[f / NRB] + (f % NRB) * 32 * PF_RB); };
+        h8 af[NFR];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) af[i] = afrag(i);
         __builtin_amdgcn_sched_barrier(0);
         uint32_t q[PF_KT][8];
         PfPair prev{0u, 0u};
+        auto mfma = [&](int m) {
+            const int f = m >> 1, kt = f / NRB, rb = f % NRB;
+            acc[rb][m & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[f], bc[kt][m & 1], acc[rb][m & 1], 0, 0, 0);
+        };
 #pragma unroll
         for (int i = 0; i < NF; ++i) {
             // the next batch's DMA instructions spread over the step (the CU's address path takes them one at a
             // time; issued together after the barrier they would stall every wave behind each other)
-            if (i % DMA_EVERY == 0 && i / DMA_EVERY < NDMA) issue_one(i / DMA_EVERY, it + NS - 1, it + NS);
-            if (i + 4 < NF && ((i + 4) & 7) < NRB) af[i + 4] = afrag(as, i + 4);
-            const int kt = i >> 3, rb = i & 7;
+            if (LAST == 0 && i % DMA_EVERY == 0 && i / DMA_EVERY < NDMA)
+                issue_one(i / DMA_EVERY, it + NS - 1, stp, it + NS, st);
+            const int m0 = i * NM / NF, m1 = (i + 1) * NM / NF;       // this pair's MFMAs: two, one, or one of two pairs
+            if (m1 > m0) {
+                if (!(m0 & 1) && (m0 >> 1) + 4 < NFR) af[(m0 >> 1) + 4] = afrag((m0 >> 1) + 4);
+                mfma(m0);
+            }
             // pair i's products after the first MFMA, pair i - 1's values after the second: no VALU instruction
             // waits on the one before it while the MFMAs run
-            if (rb < NRB) acc[rb][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bc[kt][0], acc[rb][0], 0, 0, 0);
-            const PfPair cur = pf_pair_products(w[kt], i & 7);
-            if (rb < NRB) acc[rb][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[i], bc[kt][1], acc[rb][1], 0, 0, 0);
-            if (i > 0) q[(i - 1) >> 3][(i - 1) & 7] = pf_pair_values(prev);
+            PfPair cur{0u, 0u};
+            if (LAST != 2) cur = pf_pair_products(w[i >> 3], i & 7);
+            if (m1 > m0 + 1) mfma(m0 + 1);
+            if (LAST != 2 && i > 0) q[(i - 1) >> 3][(i - 1) & 7] = pf_pair_values(prev);
             prev = cur;
             __builtin_amdgcn_sched_barrier(0);
         }
-        q[PF_KT - 1][7] = pf_pair_values(prev);
-        operands(q, bn);
+        if (LAST != 2) {
+            q[PF_KT - 1][7] = pf_pair_values(prev);
+            operands(q, bn);
+        }
     };
 #pragma unroll
     for (int rb = 0; rb < 8; ++rb)
@@ -657,9 +684,12 @@ __device__ __forceinline__ void pf_gemm(const PfTile& t, unsigned char* smem, f1
             for (int r = 0; r < 16; ++r) acc[rb][s][r] = 0.f;
     // prologue: raw words of step 0 first, then the batches that steps 0 .. NS - 2 of the loop would have issued
     // (A(0 .. NS - 2), words(1 .. NS - 1)); decode step 0
-    issue_w(0);
 #pragma unroll
-    for (int j = 0; j < NS - 1; ++j) issue(j, j + 1);
+    for (int k = NA; k < NDMA; ++k) issue_one(k, 0, 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < NS - 1; ++j)
+#pragma unroll
+        for (int k = 0; k < NDMA; ++k) issue_one(k, j, j, j + 1, j + 1);
     WAIT_VM(NDMA * (NS - 1));                                      // the step-0 words (this wave's own)
     h8 bA[PF_KT][2], bB[PF_KT][2];
     {
@@ -669,11 +699,19 @@ __device__ __forceinline__ void pf_gemm(const PfTile& t, unsigned char* smem, f1
         for (int i = 0; i < NF; ++i) q[i >> 3][i & 7] = pf_decode_pair(w[i >> 3], i & 7);
         operands(q, bA);
     }
-    static_assert(NDMA * (NS - 1) <= 63 && PF_KT % 2 == 0, "stages within the vmcnt range");
-    for (int it = 0; it < steps; it += 2) {                           // steps is even (kdim % (32 PF_KT) == 0)
-        step(it, bA, bB);
-        step(it + 1, bB, bA);
+    static_assert(NDMA * (NS - 1) <= 63 && PF_KT % 2 == 0 && NS >= 3, "stages within the vmcnt range");
+    int st = 0;
+    auto next = [&]() { st = st + 1 == NS ? 0 : st + 1; };
+    int it = 0;
+    for (; it < steps - 2; it += 2) {                                 // steps is even (kdim % (32 PF_KT) == 0)
+        step(std::integral_constant<int, 0>(), it, st, bA, bB);
+        next();
+        step(std::integral_constant<int, 0>(), it + 1, st, bB, bA);
+        next();
     }
+    step(std::integral_constant<int, 1>(), it, st, bA, bB);
+    next();
+    step(std::integral_constant<int, 2>(), it + 1, st, bB, bA);
     WAIT_VM(0);                                                       // nothing in flight when LDS is reused
     LDS_BARRIER();
 }
