@@ -8,7 +8,7 @@
 // The A rows are staged in LDS (shared by the 4 waves); each wave decodes its own trellis words straight into MFMA
 // operands, so every weight value is decoded once per tile and never goes through LDS. Calls with few rows per
 // expert run the same GEMM on 128- or 64-row parts of the segments instead (the mid- and small-tile kernels: two
-// workgroups per CU, see pf_tiles).
+// or three workgroups per CU, see pf_tiles).
 // Numerics (oracle/csrc/oracle.c mode 1 = the E3 kernels, code/fork/docs/ref/mia_exl3-fat-kernel/exl3_fat_moe.cu):
 //   gather   h13 = fp16(H(fp16(x * suh_g)) * r)                                         (exl3_fat_moe.cu:95-126)
 //   gate/up  g = (H(acc_g) * r) * svh_g, u likewise; iff L != 0: g = min(g, L), u = clamp(u, -L, L);
@@ -38,8 +38,9 @@ constexpr int PF_ASB = PF_TM * PF_RB;           // one A stage: 256 rows x 16 PF
 constexpr int PF_WWB = 512 * PF_KT;             // one wave's raw words of a step: PF_KT k tiles x 4 column tiles x 128 B
 constexpr int PF_WSB = 4 * PF_WWB;              // one raw-word stage (4 waves)
 constexpr size_t PF_LDS = (size_t)PF_NS * (PF_ASB + PF_WSB);   // 163,840 bytes (the whole LDS)
-constexpr int PF_TMS = 64;                      // rows per tile of the small-tile kernels (two per CU)
-constexpr size_t PF_LDS_S = (size_t)PF_NS * (PF_TMS * PF_RB + PF_WSB);   // 65,536 bytes
+constexpr int PF_TMS = 64;                      // rows per tile of the small-tile kernels (three per CU)
+constexpr int PF_NSS = 3;                       // their staged steps
+constexpr size_t PF_LDS_S = (size_t)PF_NSS * (PF_TMS * PF_RB + PF_WSB);  // 49,152 bytes
 constexpr int PF_TMM = 128;                     // rows per tile of the mid-tile kernels (two per CU)
 constexpr int PF_NSM = 3;                       // their staged steps
 constexpr size_t PF_LDS_M = (size_t)PF_NSM * (PF_TMM * PF_RB + PF_WSB);  // 73,728 bytes
@@ -784,7 +785,7 @@ __device__ __forceinline__ void pf_gateup_tile(const PrefillArgs& a, int s, int 
     t.btiles_n = N >> 4;
     t.bcol0 = cb * 8 + 4 * (wv & 1);
     f16v acc[8][2];
-    if (KIND == PF_SMALL) pf_gemm<E4M3, 2, PF_TMS>(t, smem, acc);
+    if (KIND == PF_SMALL) pf_gemm<E4M3, 2, PF_TMS, PF_NSS>(t, smem, acc);
     else if (KIND == PF_MID && rn <= 64) pf_gemm<E4M3, 2, PF_TMM, PF_NSM>(t, smem, acc);
     else if (KIND == PF_MID) pf_gemm<E4M3, 4, PF_TMM, PF_NSM>(t, smem, acc);
     else if (rn <= 64) pf_gemm<E4M3, 2>(t, smem, acc);              // uniform: small tiles multiply two row blocks
@@ -964,11 +965,11 @@ __global__ __launch_bounds__(PF_THREADS, 1) void pf_gateup_kernel(PrefillArgs a)
     pf_gateup_tile<E4M3, PF_LARGE>(a, s, 0, cb, smem);
 }
 
-// The same GEMM for segments of few rows: 64-row tiles with 64 KB of LDS and at most 256 registers per wave, so two
-// workgroups share a CU and one's waits are covered by the other's work (a tile's weight decode does not shrink
-// with its rows, so at ~60 rows per expert the decode, not the MFMA, bounds the GEMM).
+// The same GEMM for segments of few rows: 64-row tiles with 48 KB of LDS (three stages) and at most 168 registers per
+// wave, so three workgroups share a CU and one's waits are covered by the others' work (a tile's weight decode does not
+// shrink with its rows, so at ~60 rows per expert the decode, not the MFMA, bounds the GEMM).
 template <bool E4M3>
-__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void pf_gateup_small_kernel(
+__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(3))) void pf_gateup_small_kernel(
     PrefillArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     int s, quarter, cb;
@@ -1012,7 +1013,7 @@ __device__ __forceinline__ void pf_down_tile(const PrefillArgs& a, int s, int pa
     t.btiles_n = K >> 4;
     t.bcol0 = cb * 16 + 4 * wv;
     f16v acc[8][2];
-    if (KIND == PF_SMALL) pf_gemm<E4M3, 2, PF_TMS>(t, smem, acc);
+    if (KIND == PF_SMALL) pf_gemm<E4M3, 2, PF_TMS, PF_NSS>(t, smem, acc);
     else if (KIND == PF_MID && rn <= 64) pf_gemm<E4M3, 2, PF_TMM, PF_NSM>(t, smem, acc);
     else if (KIND == PF_MID) pf_gemm<E4M3, 4, PF_TMM, PF_NSM>(t, smem, acc);
     else if (rn <= 64) pf_gemm<E4M3, 2, PF_TM, PF_NS, ACOH>(t, smem, acc);
@@ -1100,7 +1101,7 @@ __global__ __launch_bounds__(PF_THREADS, 1) void pf_down_kernel(PrefillArgs a) {
 }
 
 template <bool E4M3>
-__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void pf_down_small_kernel(
+__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(3))) void pf_down_small_kernel(
     PrefillArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     int s, quarter, cb;
@@ -1121,7 +1122,7 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 // ------------------------------------------------------------------------------------------------ one-launch schedule
 
 // Every gate/up and down tile of a call in one launch of one workgroup per CU (256-row tiles; two per CU for the
-// 128- and 64-row part tiles, KIND below). The segments are dealt to eight ticket queues (segment s to queue s % 8, as the separate launches deal them to the
+// 128-row and three for the 64-row part tiles, KIND below). The segments are dealt to eight ticket queues (segment s to queue s % 8, as the separate launches deal them to the
 // XCDs), each ordered by pf_sched_item over its own segments; a workgroup takes tickets from its own XCD's queue
 // (the XCC_ID register), so a segment's column blocks share that XCD's L2 for their A rows, and once that queue is
 // empty from the other queues in turn. A gate/up item stores its h2 rows device-coherent (written through to the
@@ -1141,7 +1142,7 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 enum { PF_SCHED_E3 = 0, PF_SCHED_E4M3_16 = 1, PF_SCHED_E4M3 = 2 };
 constexpr int PF_SCHED_POLLS = 1 << 20;
 // KIND: the call's tile kind (PF_LARGE: 256-row segments, one workgroup per CU; PF_MID / PF_SMALL: the segments'
-// 128- or 64-row parts, two workgroups per CU). A queue's units are its (segment, part) pairs, every segment's first
+// 128- or 64-row parts, two or three workgroups per CU). A queue's units are its (segment, part) pairs, every segment's first
 // part first; a part past its segment's rows holds no tile, so its items only take their tickets. Each unit has its
 // own count (segment s, part p: word PF_SCHED_HEAD + s * parts + p).
 template <int MODE, int KIND>
@@ -1235,7 +1236,7 @@ __global__ __launch_bounds__(PF_THREADS, 1) void pf_sched_kernel(PrefillArgs a) 
     pf_sched_body<MODE, PF_LARGE>(a, smem);
 }
 template <int MODE, int KIND>
-__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(2))) void pf_sched_part_kernel(
+__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(KIND == PF_SMALL ? 3 : 2))) void pf_sched_part_kernel(
     PrefillArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     pf_sched_body<MODE, KIND>(a, smem);
@@ -1644,19 +1645,23 @@ int prefill_setup() {
 
 // Which grouped GEMMs a call runs. Tiles of few rows are bound by the weight decode on the VALU, and the 256-row
 // kernels run one workgroup per CU (160 KB of staging, 256 accumulator registers), which leaves the VALU idle at
-// every barrier and load wait. The mid- and small-tile kernels run two workgroups per CU, at the price of decoding
-// a segment's weights once per 128-row half or 64-row quarter. Measured at 288 experts, top-8 (E3 numerics /
-// trellis-sourced e4m3), against the 256-row kernels:
-//   T = 2048 (~57 rows per expert):  mid 27 % faster / small 18 % faster (mid 3 % slower);
-//   T = 4096 (~114 rows):            mid 29 % faster / mid 21 % faster (small 3 % slower);
-//   T = 6144 (~171 rows):            mid 4 % slower;
-//   T = 8192 (~228 rows):            mid 8 % slower, small 47 % slower; Zipf-skewed routing: mid 4 % faster.
-// Hence: P <= 64 n: mid (small for e4m3); P <= 128 n: mid; larger calls: the 256-row kernels. P is the pairs
-// expected on this call's experts: with an expert map only the share n / n_global of the routed ones (144 of 288
-// experts, T = 4289, Zipf routing, 119 rows per expert: mid 823 us, 256-row tiles 931). "hybrid" splits a
-// call by segment size (segments of at most PF_SMALL_ROWS rows on the small tiles, larger ones on the 256-row
-// tiles). The environment variable MI355MOE_PREFILL_TILES = "small", "mid", "large" or "hybrid" forces a choice;
-// all give bit-identical results (a row's arithmetic does not depend on the tile that holds it).
+// every barrier and load wait. The mid-tile kernels run two workgroups per CU and the small-tile ones three (VALU busy
+// 76 and 84 %), at the price of decoding a segment's weights once per 128-row half or 64-row quarter. Measured at top-8
+// (288 experts, hidden 4096, intermediate 1024 unless given; E3 numerics / trellis-sourced e4m3), us per call:
+//   T = 600 (17 rows per expert):   mid 770, small 771; Zipf-skewed routing mid 857, small 846
+//   T = 1024 - 1100 (28 - 31 rows): mid 789 / 874, small 749 / 844; Zipf mid 933, small 950; intermediate 256 mid 268,
+//                                   small 274; intermediate 512, hidden 2048 mid 256, small 248
+//   T = 1791 (50 rows):             mid 837 / 976, small 818 / 967; Zipf mid 1075, small 1132; intermediate 256,
+//                                   T = 1700 mid 310, small 325
+//   T = 2048 (57 rows):             mid 870 / 976, small 880 / 1036 (T = 2000), 256-row tiles about 1110 / 1366
+//   T = 4096 (~114 rows):           mid 29 % / 21 % faster than the 256-row tiles
+//   T = 6144 (~171 rows):           mid 4 % slower; T = 8192 (~228 rows): mid 8 % slower (Zipf: mid 4 % faster).
+// Hence: P <= 36 n: small; P <= 128 n: mid; larger calls: the 256-row kernels. P is the pairs expected on this call's
+// experts: with an expert map only the share n / n_global of the routed ones (144 of 288 experts, T = 4289, Zipf
+// routing, 119 rows per expert: mid 823 us, 256-row tiles 931). "hybrid" splits a call by segment size (segments of at
+// most PF_SMALL_ROWS rows on the small tiles, larger ones on the 256-row tiles). The environment variable
+// MI355MOE_PREFILL_TILES = "small", "mid", "large" or "hybrid" forces a choice; all give bit-identical results (a
+// row's arithmetic does not depend on the tile that holds it).
 constexpr int PF_SMALL_ROWS = 128;
 enum { PF_TILES_SMALL = 1, PF_TILES_LARGE = 2, PF_TILES_BOTH = 3, PF_TILES_MID = 4 };
 static int pf_tiles(const PrefillArgs& a) {
@@ -1667,7 +1672,7 @@ static int pf_tiles(const PrefillArgs& a) {
     if (f && !strcmp(f, "hybrid")) return PF_TILES_BOTH;
     if (a.n <= 0) return PF_TILES_LARGE;
     const int64_t P = a.pairs_local > 0 ? a.pairs_local : a.P, n = a.n;
-    if (P <= 64 * n) return a.e4m3 ? PF_TILES_SMALL : PF_TILES_MID;
+    if (P <= 36 * n) return PF_TILES_SMALL;
     return P <= 128 * n ? PF_TILES_MID : PF_TILES_LARGE;
 }
 
@@ -1715,7 +1720,7 @@ int launch_prefill(const PrefillArgs& a0, hipStream_t st, int kernels) {
     if (sched) {
         a.small_rows = 0;
         const int parts = tiles == PF_TILES_SMALL ? 4 : tiles == PF_TILES_MID ? 2 : 1;
-        const int per_cu = parts > 1 ? 2 : 1;
+        const int per_cu = parts > 2 ? 3 : parts > 1 ? 2 : 1;
         const int64_t items = (int64_t)std::max(a.S_cap, 0) * parts * ((a.N >> 7) + (a.K >> 8));
         const dim3 grid((unsigned)std::min<int64_t>((int64_t)per_cu * pf_device_cus(), items)), blk(PF_THREADS);
         const int mode = !f8 ? 0 : a.down16 ? 1 : 2;
