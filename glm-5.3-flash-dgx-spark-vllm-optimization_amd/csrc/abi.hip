@@ -66,14 +66,6 @@ int sched_lag() {
     return v ? std::max(0, atoi(v)) : 0;
 }
 
-// Whether a decode call of a layer with one w13 suh rotates its tokens' rows first, in a launch of their own: every
-// gate/up workgroup then copies its segment's staged rows instead of rotating them (each of the N / 128 column blocks
-// of each of a token's experts rotated it again: 23 % of the kernel's VALU instructions at 9 rows per expert). The
-// launch costs 4 - 6 us, which 1.5 pairs per expert pay for (288 experts, hidden 4096, intermediate 1024, rotated first
-// / in the workgroups: T = 8 118 / 115 us, 24 260 / 257, 32 303 / 304, 64 399 / 406, 128 479 / 498, 333 539 / 594,
-// 500 658 / 732).
-bool rotate_first(int64_t P, int64_t n) { return 2 * P >= 3 * n; }
-
 struct DecodePlan {
     int rmax, seg, S_cap, sk_gu, sk_dn, kch_gu, kch_dn;
 };
@@ -576,7 +568,9 @@ static int prep_decode(const mi355moe_exl3_layer* layer, const void* x, int x_dt
     d.kch_gu = p.kch_gu;
     d.kch_dn = p.kch_dn;
     d.shared_suh = shared_flag(layer);
-    if (tok_rows_flag(layer) && rotate_first(P, n)) d.xrot = reinterpret_cast<uint16_t*>(d.contrib);   // [T][K] of [P][2K]
+    // (not where K is split, for a handful of segments, nor up to 4 tokens: nothing to gain there, +0.2 us of 40)
+    if (tok_rows_flag(layer) && p.sk_gu == 1 && T > 4)
+        d.xrot = reinterpret_cast<uint16_t*>(d.contrib);             // [T][K] halves of [P][K] floats
     d.limit = limit;
     d.out = out;
     d.odt = dt_w(out_dtype);
@@ -584,6 +578,18 @@ static int prep_decode(const mi355moe_exl3_layer* layer, const void* x, int x_dt
     d.accumulate = 0;
     d.topk = (int)topk;
     return 0;
+}
+
+// A decode call of a layer with one w13 suh rotates its tokens' rows once, in additional workgroups of its first route
+// kernel, and every gate/up workgroup copies its segment's staged rows instead of rotating them (each of the N / 128
+// column blocks of each of a token's experts rotated it again: 23 % of the kernel's VALU instructions at 9 rows per
+// expert). Layer or routed call with / without it (288 experts, hidden 4096, top-8, intermediate 1024; us): T = 8
+// 105.8 / 107.8, 24 245 / 252, 64 385 / 395, 333 520 / 572, 500 631 / 704; skewed routing, intermediate 256: T = 12
+// 60.1 / 68.9, 47 78.9 / 92.1. (A launch of its own costs 4 - 6 us, more than it gains up to T = 24.)
+static void rotate_with_route(DecodeWs& w) {
+    if (!w.da.xrot) return;
+    w.ra.rot = RotateArgs{w.da.x, w.da.xdt, w.da.x_stride, w.da.T, w.da.K, w.da.wt.g_suh, w.da.xrot};
+    w.da.xrot_done = 1;
 }
 
 // The grouped (prefill) tier over 256-row expert tiles for validated arguments: E3's fp16 numerics, or with e4m3 the
@@ -714,6 +720,7 @@ int mi355moe_moe_forward_ids_opt(const mi355moe_exl3_layer* layer, const void* x
     r.wdt = dt_w(weights_dtype);
     r.emap = expert_map;
     r.n_global = expert_map ? n_global : 0;
+    if ((stages & MI355MOE_STAGE_ROUTE) && (stages & MI355MOE_STAGE_GATEUP)) rotate_with_route(w);
     if (stages & MI355MOE_STAGE_ROUTE)
         if (int rc = launch_route(r, stream)) return rc_launch(rc);
     w.da.out_accumulate = (options & MI355MOE_OPT_ACCUMULATE) ? 1 : 0;
@@ -1004,6 +1011,7 @@ int mi355moe_moe_layer(const mi355moe_exl3_layer* layer, const void* x, int x_dt
         r.wdt = dt_w(MI355MOE_F32);
         r.emap = nullptr;
         r.n_global = 0;
+        rotate_with_route(w);
         const int rc = router_w ? launch_router_route(static_cast<const uint16_t*>(x), x_stride,
                                                       static_cast<const uint16_t*>(router_w), (int)K, lg, (int)T,
                                                       (int)E, bias, (int)topk, routed_scale, renormalize ? 1 : 0, ids,

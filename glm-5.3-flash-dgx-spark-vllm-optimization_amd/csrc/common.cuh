@@ -269,6 +269,21 @@ __device__ __forceinline__ int ld_coherent(const int* p) {
     return __hip_atomic_load(const_cast<int*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Store a lane's four packed pairs (k pairs 4h .. 4h + 3 of 16-group g, lane c = 2g + h) at their permuted positions
+// with one 16-byte store: the lanes c, c ^ 1 of a group own its 32 bytes interleaved (storage pair 2m + h = the lane's
+// pair m), so they swap two pairs (DPP lane ^ 1) and lane h then writes storage pairs 4h .. 4h + 3 contiguously.
+// grp: the 16-group's first element.
+__device__ __forceinline__ u32x4 pf_group_vec(const uint32_t (&wm)[4], int c) {
+    const bool hi = c & 1;
+    const uint32_t s0 = hi ? wm[0] : wm[2], s1 = hi ? wm[1] : wm[3];
+    const uint32_t r0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)s0, 0xB1, 0xF, 0xF, true);   // lane ^ 1
+    const uint32_t r1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)s1, 0xB1, 0xF, 0xF, true);
+    return hi ? u32x4{r0, wm[2], r1, wm[3]} : u32x4{wm[0], r0, wm[1], r1};
+}
+__device__ __forceinline__ void pf_store_group(_Float16* grp, const uint32_t (&wm)[4], int c) {
+    *reinterpret_cast<u32x4*>(grp + 8 * (c & 1)) = pf_group_vec(wm, c);
+}
+
 // ---------------------------------------------------------------------------------------------- LDS staging
 
 // Wave instruction: 64 lanes x 16 bytes, lane l -> LDS bytes lds_wave + 16 l (global_load_lds_dwordx4). Written as

@@ -18,8 +18,6 @@
 //            suh_d)) * r)
 //   down     v = H(sum_n xd Wq_d) * (r * w16) * svh_d                   (exl3.cu:455-496)
 //   combine  out[t] = sum over the token's slots in slot order (exl3.cu:815-864), or fp32 atomics (accumulate mode)
-#include <cstring>
-
 #include "common.cuh"
 #include "mi355moe_internal.h"
 
@@ -1013,18 +1011,9 @@ int launch_decode(const DecodeArgs& a0, int rmax, hipStream_t st, int kernels) {
         const bool multi = gateup_passes(rmax, a.kch_gu, a.shared_suh != 0, a.lds_gu) > 1;
         auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(GU_WAVES * 64), lds, st, a); };
         if (a.shared_suh && a.xrot) {
-            PrefillArgs g;
-            memset(&g, 0, sizeof(g));
-            g.wt = a.wt;
-            g.n = a.n;
-            g.K = a.K;
-            g.T = a.T;
-            g.x = a.x;
-            g.xdt = a.xdt;
-            g.x_stride = a.x_stride;
-            g.tok_rows = 1;
-            g.h13 = a.xrot;
-            if (launch_gather_tokens(g, st)) return -1;
+            if (!a.xrot_done &&
+                launch_rotate(RotateArgs{a.x, a.xdt, a.x_stride, a.T, a.K, a.wt.g_suh, a.xrot}, st))
+                return -1;
             if (multi) d4 ? go(dec_gateup_kernel<4, true, true, true>) : go(dec_gateup_kernel<2, true, true, true>);
             else d4 ? go(dec_gateup_kernel<4, true, false, true>) : go(dec_gateup_kernel<2, true, false, true>);
         } else if (a.shared_suh) {

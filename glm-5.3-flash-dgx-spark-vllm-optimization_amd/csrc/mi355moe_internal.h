@@ -10,6 +10,17 @@ enum DType { DT_F32 = 0, DT_F16 = 1, DT_BF16 = 2 };
 constexpr int ROUTE_SMALL_MAX_P = 1024;   // pairs the one-block permutation handles
 
 // Permutation of P = T * topk routed pairs into expert order.
+// Rotated token rows for a layer whose experts share one w13 suh: out[t][k] = fp16(H(fp16(x[t] * suh)) * r), fp16, the
+// columns of every 16-group in the staged order 0, 1, 8, 9, 2, 3, ... (out == nullptr: none)
+struct RotateArgs {
+    const void* x;
+    int xdt;
+    int64_t x_stride;       // elements
+    int T, K;
+    const int64_t* suh;     // device pointer table (entry 0 is read)
+    uint16_t* out;          // [T][K]
+};
+
 struct RouteArgs {
     const void* ids;        // [P] int32 or int64 router ids
     int ids64;
@@ -37,6 +48,7 @@ struct RouteArgs {
     // split-K arrival counters of the kernels that follow, zeroed by the first route kernel of the call
     unsigned* zero;
     int64_t zero_words;
+    RotateArgs rot;         // rotated by additional workgroups of the call's first route kernel
 };
 
 // Pointer tables of one layer's experts: device arrays of n int64 device addresses.
@@ -61,8 +73,9 @@ struct DecodeArgs {
     int xdt;                // DT_F16 or DT_BF16
     int64_t x_stride;       // elements
     uint16_t* xrot;         // optional, layers whose experts share one w13 suh: [T][K] fp16, the tokens' rotated rows
-                            // in the staged order (xa_pos), written before gate/up by launch_decode (may alias
-                            // contrib, which the down kernel fills after the last read)
+                            // in the staged order (xa_pos); may alias contrib, which the down kernel fills after the
+                            // last read
+    int xrot_done;          // the call's route kernel has written them (0: launch_decode does, ahead of gate/up)
     // routing tables (sorted position order)
     const int* tok;
     const uint16_t* w16;
@@ -314,7 +327,7 @@ int launch_decode(const DecodeArgs& a, int rmax, hipStream_t st, int kernels = 7
 size_t decode_lds_gateup(int rmax, int kr, int shared_suh);
 size_t decode_lds_down(int rmax, int kr);
 constexpr size_t DECODE_LDS_MAX = 81920;   // two 512-thread workgroups per CU
-int launch_gather_tokens(const PrefillArgs& a, hipStream_t st);
+int launch_rotate(const RotateArgs& a, hipStream_t st);
 int launch_dequant(const uint16_t* trellis, int kt, int nt, uint16_t* wq, hipStream_t st);
 int launch_sigmoid(const float* g, int64_t n, int variant, float* out, hipStream_t st);
 int launch_rot_in(const void* x, int xdt, int64_t x_stride, const int* tok, const int* pe, const int64_t* suh_tab,

@@ -60,21 +60,7 @@ __host__ __device__ constexpr int pf_epi_blocks(int kind) {
 // go straight into MFMA operands (8 consecutive k slots per lane) and the activations match them slot for slot.
 __device__ __forceinline__ int pf_kperm_pair(int j) { return 2 * (j & 3) + (j >> 2); }
 
-// Store a lane's four packed pairs (k pairs 4h .. 4h + 3 of 16-group g, lane c = 2g + h) at their permuted positions
-// with one 16-byte store: the lanes c, c ^ 1 of a group own its 32 bytes interleaved (storage pair 2m + h = the lane's
-// pair m), so they swap two pairs (DPP lane ^ 1) and lane h then writes storage pairs 4h .. 4h + 3 contiguously.
-// grp: the 16-group's first element.
-__device__ __forceinline__ u32x4 pf_group_vec(const uint32_t (&wm)[4], int c) {
-    const bool hi = c & 1;
-    const uint32_t s0 = hi ? wm[0] : wm[2], s1 = hi ? wm[1] : wm[3];
-    const uint32_t r0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)s0, 0xB1, 0xF, 0xF, true);   // lane ^ 1
-    const uint32_t r1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)s1, 0xB1, 0xF, 0xF, true);
-    return hi ? u32x4{r0, wm[2], r1, wm[3]} : u32x4{wm[0], r0, wm[1], r1};
-}
-__device__ __forceinline__ void pf_store_group(_Float16* grp, const uint32_t (&wm)[4], int c) {
-    *reinterpret_cast<u32x4*>(grp + 8 * (c & 1)) = pf_group_vec(wm, c);
-}
-// The same as one device-coherent store, for rows that workgroups on other XCDs read in the same launch: r over the
+// pf_store_group as one device-coherent store, for rows that workgroups on other XCDs read in the same launch: r over the
 // row block, grp_off the 16-group's byte offset in it.
 __device__ __forceinline__ void pf_store_group_coh(__amdgpu_buffer_rsrc_t r, int grp_off, const uint32_t (&wm)[4],
                                                    int c) {
@@ -1674,12 +1660,6 @@ static int pf_tiles(const PrefillArgs& a) {
     const int64_t P = a.pairs_local > 0 ? a.pairs_local : a.P, n = a.n;
     if (P <= 36 * n) return PF_TILES_SMALL;
     return P <= 128 * n ? PF_TILES_MID : PF_TILES_LARGE;
-}
-
-// One rotated row per token (a.tok_rows) into h13.
-int launch_gather_tokens(const PrefillArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL(pf_gather_kernel, dim3(std::max(1, std::min(4096, (a.T + 3) / 4))), dim3(256), 0, st, a);
-    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int launch_prefill(const PrefillArgs& a0, hipStream_t st, int kernels) {

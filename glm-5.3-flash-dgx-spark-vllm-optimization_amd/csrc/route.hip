@@ -496,6 +496,65 @@ __device__ void build_segments(const int* cnt, const int* start, int n, int R, i
     if (threadIdx.x == 0) nseg_out[0] = run < S_cap ? run : S_cap;
 }
 
+// Rotated token rows (RotateArgs), in tasks of one wave: token t, four 128-blocks (16 lanes per block, 8 consecutive
+// elements per lane). Wave w of nw takes tasks w, w + nw, ... The product with r is rounded to fp32 before fp16 (as the
+// oracle has it): without the barrier the compiler fuses the two in some call sites and not in others.
+__device__ void rotate_tasks(const RotateArgs& a, int w, int nw) {
+    const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
+    const int nb = a.K >> 7, np = (nb + 3) >> 2;
+    const uint16_t* suh = reinterpret_cast<const uint16_t*>(a.suh[0]);
+    for (int task = w; task < a.T * np; task += nw) {
+        const int t = task / np, blk = 4 * (task - t * np) + q;
+        if (blk >= nb) continue;                                     // (whole 16-lane groups)
+        const int col = 128 * blk + 8 * c;
+        const uint16_t* xp = reinterpret_cast<const uint16_t*>(a.x) + (size_t)t * a.x_stride + col;
+        uint32_t xv[4], sv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            xv[i] = *reinterpret_cast<const uint32_t*>(xp + 2 * i);
+            sv[i] = *reinterpret_cast<const uint32_t*>(suh + col + 2 * i);
+        }
+        float p[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool bf = a.xdt == DT_BF16;
+            const _Float16 h0 = bf ? (_Float16)__builtin_bit_cast(float, xv[i] << 16) : u16_as_h(xv[i] & 0xFFFFu);
+            const _Float16 h1 = bf ? (_Float16)__builtin_bit_cast(float, xv[i] & 0xFFFF0000u) : u16_as_h(xv[i] >> 16);
+            p[2 * i] = (float)(_Float16)(h0 * u16_as_h(sv[i] & 0xFFFFu));
+            p[2 * i + 1] = (float)(_Float16)(h1 * u16_as_h(sv[i] >> 16));
+        }
+        fwht128_x16s(p, lane);
+        const float hr = HAD_R * fwht_sign(lane);
+        uint32_t wm[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            float v0 = p[2 * m] * hr, v1 = p[2 * m + 1] * hr;
+            asm volatile("" : "+v"(v0), "+v"(v1));
+            wm[m] = __builtin_bit_cast(uint32_t, h2{(_Float16)v0, (_Float16)v1});
+        }
+        pf_store_group(reinterpret_cast<_Float16*>(a.out) + (size_t)t * a.K + 128 * blk + 16 * (c >> 1), wm, c);
+    }
+}
+// The rotation as the workgroups past `first` of a route launch (one wave per task), and their number.
+__device__ __forceinline__ bool rotate_blocks(const RotateArgs& a, int first) {
+    if ((int)blockIdx.x < first) return false;
+    const int waves = blockDim.x >> 6;
+    rotate_tasks(a, ((int)blockIdx.x - first) * waves + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)),
+                 ((int)gridDim.x - first) * waves);
+    return true;
+}
+static unsigned rotate_grid(const RotateArgs& a, int threads) {
+    if (!a.out || a.T <= 0) return 0;
+    const int64_t tasks = (int64_t)a.T * (((a.K >> 7) + 3) / 4), per = threads / 64;
+    return (unsigned)std::min<int64_t>(1024, (tasks + per - 1) / per);
+}
+__global__ __launch_bounds__(256) void rotate_kernel(RotateArgs a) { rotate_blocks(a, 0); }
+
+int launch_rotate(const RotateArgs& a, hipStream_t st) {
+    if (const unsigned g = rotate_grid(a, 256)) hipLaunchKernelGGL(rotate_kernel, dim3(g), dim3(256), 0, st, a);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 // Zeroes this call's split-K arrival counters (a grid-stride fill by the first kernel of the call).
 __device__ __forceinline__ void zero_counters(const RouteArgs& a) {
     if (!a.zero) return;
@@ -638,6 +697,7 @@ __device__ void route_wave64(const RouteArgs& a) {
 template <typename IT>
 __global__ __launch_bounds__(1024) void route_small_kernel(RouteArgs a) {
     extern __shared__ int sh[];
+    if (rotate_blocks(a.rot, 1)) return;
     route_small_body<IT>(a, sh);
 }
 
@@ -909,6 +969,7 @@ __global__ __launch_bounds__(MAXT) void topk_route_kernel(const float* __restric
                                                           int renorm, int32_t* __restrict__ ids,
                                                           float* __restrict__ wts, RouteArgs a) {
     extern __shared__ int sh[];
+    if (rotate_blocks(a.rot, 1)) return;
     topk_route_body<J, false>(logits, T, E, bias, topk, scale, renorm, ids, wts, a, sh);
 }
 
@@ -928,6 +989,8 @@ __global__ __launch_bounds__(MAXT) void router_route_kernel(const uint16_t* __re
                                                             RouteArgs a, unsigned* arrivals) {
     extern __shared__ int sh[];
     __shared__ int last;
+    const unsigned nrb = (E + RR_EXPERTS - 1) / RR_EXPERTS;           // the router's workgroups, then the rotation's
+    if (rotate_blocks(a.rot, (int)nrb)) return;
     logits_body<true, RR_EXPERTS, true>(x, x_stride, w, T, K, E, RR_EXPERTS * blockIdx.x, logits);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -937,7 +1000,7 @@ __global__ __launch_bounds__(MAXT) void router_route_kernel(const uint16_t* __re
     // workspace not zero-filled before its first use) still elects one workgroup per call and the tables are always
     // rebuilt; the last arrival of each level returns its word to zero.
     if (threadIdx.x == 0) {
-        const unsigned G = min(RR_GROUPS, gridDim.x), g = blockIdx.x % G, size = (gridDim.x - 1 - g) / G + 1;
+        const unsigned G = min(RR_GROUPS, nrb), g = blockIdx.x % G, size = (nrb - 1 - g) / G + 1;
         unsigned* gw = arrivals + 64 * (g + 1);
         int l = 0;
         if ((__hip_atomic_fetch_add(gw, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u) % size == 0u) {
@@ -1152,6 +1215,7 @@ __global__ __launch_bounds__(ROUTE_BLK) void route_hist_kernel(RouteArgs a) {
     extern __shared__ int cnt[];
     const IT* ids = reinterpret_cast<const IT*>(a.ids);
     zero_counters(a);
+    if (rotate_blocks(a.rot, (a.P + ROUTE_BLK - 1) / ROUTE_BLK)) return;
     for (int e = threadIdx.x; e <= a.n; e += blockDim.x) cnt[e] = 0;
     __syncthreads();
     const int j = blockIdx.x * ROUTE_BLK + threadIdx.x;
@@ -1381,10 +1445,10 @@ int launch_topk_route(const float* logits, int T, int E, const float* bias, int 
         attr = true;
     }
     if (E <= 320)
-        hipLaunchKernelGGL(topk_route_kernel<5>, dim3(1), dim3(1024), shm, st, logits, T, E, bias, topk, scale, renorm,
+        hipLaunchKernelGGL(topk_route_kernel<5>, dim3(1 + rotate_grid(a.rot, 1024)), dim3(1024), shm, st, logits, T, E, bias, topk, scale, renorm,
                            ids, wts, a);
     else
-        hipLaunchKernelGGL((topk_route_kernel<16, 512>), dim3(1), dim3(512), shm, st, logits, T, E, bias, topk, scale,
+        hipLaunchKernelGGL((topk_route_kernel<16, 512>), dim3(1 + rotate_grid(a.rot, 512)), dim3(512), shm, st, logits, T, E, bias, topk, scale,
                            renorm, ids, wts, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
@@ -1404,7 +1468,7 @@ int launch_router_route(const uint16_t* x, int64_t x_stride, const uint16_t* w, 
             return -1;
         attr = true;
     }
-    const dim3 grid((E + RR_EXPERTS - 1) / RR_EXPERTS);
+    const dim3 grid((E + RR_EXPERTS - 1) / RR_EXPERTS + rotate_grid(a.rot, 64 * nw));
     if (E <= 320)
         hipLaunchKernelGGL(router_route_kernel<5>, grid, dim3(64 * nw), shm, st, x, x_stride, w, T, K, E, logits,
                            bias, topk, scale, renorm, ids, wts, a, arrivals);
@@ -1427,14 +1491,15 @@ int launch_route_counts(const int64_t* counts64, const int64_t* token_sorted, co
 int launch_route(const RouteArgs& a, hipStream_t st) {
     if (a.P <= ROUTE_SMALL_MAX_P) {
         const size_t shm = (size_t)(a.P + 2 * (a.n + 1)) * sizeof(int);
-        if (a.ids64) hipLaunchKernelGGL(route_small_kernel<int64_t>, dim3(1), dim3(1024), shm, st, a);
-        else hipLaunchKernelGGL(route_small_kernel<int32_t>, dim3(1), dim3(1024), shm, st, a);
+        if (a.ids64) hipLaunchKernelGGL(route_small_kernel<int64_t>, dim3(1 + rotate_grid(a.rot, 1024)), dim3(1024), shm, st, a);
+        else hipLaunchKernelGGL(route_small_kernel<int32_t>, dim3(1 + rotate_grid(a.rot, 1024)), dim3(1024), shm, st, a);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
     const int nblk = (a.P + ROUTE_BLK - 1) / ROUTE_BLK;
     const size_t shm1 = (size_t)(a.n + 1) * sizeof(int);
-    if (a.ids64) hipLaunchKernelGGL(route_hist_kernel<int64_t>, dim3(nblk), dim3(ROUTE_BLK), shm1, st, a);
-    else hipLaunchKernelGGL(route_hist_kernel<int32_t>, dim3(nblk), dim3(ROUTE_BLK), shm1, st, a);
+    const unsigned hist = nblk + rotate_grid(a.rot, ROUTE_BLK);
+    if (a.ids64) hipLaunchKernelGGL(route_hist_kernel<int64_t>, dim3(hist), dim3(ROUTE_BLK), shm1, st, a);
+    else hipLaunchKernelGGL(route_hist_kernel<int32_t>, dim3(hist), dim3(ROUTE_BLK), shm1, st, a);
     const size_t shm_lds = (size_t)(a.n + 1) * (2 + nblk) * sizeof(int);
     static bool lds_attr = false;
     if (nblk <= 64 && shm_lds <= ROUTE_SCAN_LDS_MAX && !lds_attr) {

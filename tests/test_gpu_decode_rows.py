@@ -40,9 +40,26 @@ def test_rows_per_segment(cuda, K, N, shared, rows):
     _check(cuda, K, N, rows, shared_suh=shared)
 
 
-# one w13 suh for every expert: from 4 rows here (1.5 pairs per expert) the rows are rotated once per token and copied,
-# by LDS DMA where a pass is whole 512-k pieces, by register loads where it is not or where the rows are duplicated
+# one w13 suh for every expert: calls of more than 4 rows rotate them once per token (with the call's first route launch,
+# or, GATEUP staged alone, in a launch of its own) and the workgroups copy them, by LDS DMA where a pass is whole 512-k pieces, by register loads where it is not or where the rows are duplicated
 @pytest.mark.parametrize("K,N", [(4096, 256), (8192, 128), (6144, 128), (768, 128), (256, 128), (10240, 128)])
-@pytest.mark.parametrize("rows", [3, 4, 5, 9, 16, 17, 35])
+@pytest.mark.parametrize("rows", [3, 4, 5, 9, 16, 17, 35, 520])
 def test_rows_rotated_once(cuda, K, N, rows):
     _check(cuda, K, N, rows, uniform_suh=True)
+
+
+@pytest.mark.parametrize("rows", [5, 40])
+def test_rows_rotated_by_stage(cuda, rows):
+    """The routing staged alone, then the experts (whose rotation is then a launch of its own): bit-equal to one call."""
+    from mi355moe import _lib, ops, synthetic
+    print(f"decode by stage rows={rows}", flush=True)
+    ex = synthetic.calibrated_layer(5, 1280, 128, seed=11, device=cuda, uniform_suh=True)
+    x = synthetic.activations(rows, 1280, seed=12, device=cuda)
+    ids = torch.stack([torch.zeros(rows, dtype=torch.int32), 1 + torch.arange(rows, dtype=torch.int32) % 4], 1).to(cuda)
+    w = synthetic.softmax_weights(rows, 2, seed=13, device=cuda)
+    kw = dict(out_dtype=torch.float32, path=_lib.PATH_DECODE)
+    whole = ops.moe_forward_ids(ex, x, ids, w, **kw)
+    out = torch.zeros_like(whole)
+    ops.moe_forward_ids(ex, x, ids, w, out=out, stages=_lib.STAGE_ROUTE, **kw)
+    ops.moe_forward_ids(ex, x, ids, w, out=out, stages=_lib.STAGE_GATEUP | _lib.STAGE_DOWN | _lib.STAGE_COMBINE, **kw)
+    assert torch.equal(out, whole)
