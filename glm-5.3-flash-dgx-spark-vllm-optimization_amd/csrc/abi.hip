@@ -191,7 +191,7 @@ struct Fp8Ws {
     size_t bytes;
 };
 
-// Layout of the e4m3 path's workspace: route tables (64-row segments), quantised activations, SwiGLU output and
+// Layout of the e4m3 path's workspace: route tables (64-row segments, 8-row ones for few tokens), quantised activations, SwiGLU output and
 // its quantisation, the per-pair fp32 contributions.
 void carve_fp8(void* ws, int64_t P, int64_t T, int64_t n, int64_t K, int64_t N, Fp8Ws& w, int& S_cap) {
     Carve c(ws);
@@ -199,7 +199,7 @@ void carve_fp8(void* ws, int64_t P, int64_t T, int64_t n, int64_t K, int64_t N, 
     Fp8Args& f = w.fa;
     memset(&r, 0, sizeof(r));
     memset(&f, 0, sizeof(f));
-    S_cap = (int)(std::min(P, n) + (P + FP8_TM - 1) / FP8_TM);
+    S_cap = (int)(std::min(P, n) + (P + fp8_seg_rows(T) - 1) / fp8_seg_rows(T));
     r.tok = c.take<int>(P);
     r.w16 = c.take<uint16_t>(P);
     r.w32 = c.take<float>(P);
@@ -1681,7 +1681,7 @@ int mi355moe_fp8_moe_forward_ids(const mi355moe_fp8_layer* layer, const void* x,
     r.topk = (int)topk;
     r.n = (int)n;
     r.R = 1 << 30;
-    r.seg = FP8_TM;
+    r.seg = fp8_seg_rows(T);
     r.S_cap = S_cap;
     Fp8Args& f = w.fa;
     f.n = (int)n;

@@ -401,6 +401,154 @@ __global__ __launch_bounds__(256) void fp8_down_kernel(Fp8Args a) {
     }
 }
 
+// ------------------------------------------------------------------------------------------------ few tokens
+
+// The two GEMMs for segments of at most FP8_FEW rows (fp8_seg_rows): 128 weight rows and FP8_FEW activation rows per
+// stage (17 KB, three workgroups per CU). Every wave copies 32 weight rows and all the activation rows (the four waves
+// write the same bytes), so all wait for the same number of loads. MFMA row r takes activation row r % FP8_FEW; only
+// rows below the segment's are stored. A row's arithmetic is that of the 64-row kernels.
+constexpr int FEW_ROWS = 128 + FP8_FEW;
+constexpr int FEW_INST = 128 / 8 / 4 + 1;
+struct FewTile {
+    const uint8_t* src[FEW_INST];
+    int lds[FEW_INST];
+};
+__device__ __forceinline__ void few_issue(const FewTile& t, unsigned char* st, int kb) {
+#pragma unroll
+    for (int j = 0; j < FEW_INST - 1; ++j) dma16_nt(t.src[j] + (size_t)kb * 128, st + t.lds[j]);
+    dma16(t.src[FEW_INST - 1] + (size_t)kb * 128, st + t.lds[FEW_INST - 1]);
+}
+// The pipeline of nkb blocks in three stages: first(kb == 0) publishes the staged scales, acc += block sums of this wave's
+// 32 weight rows (stage rows 32 wv ..) times scl[kb].
+template <typename First>
+__device__ __forceinline__ void few_gemm(const FewTile& t, unsigned char* st, int nkb, int wv, int lane, const float* scl,
+                                         const First& first, f32x16& acc) {
+    const int h = lane >> 5, c = lane & 31;
+    constexpr int SB = FEW_ROWS * 128;
+    auto step = [&](int cur, int nxt, int kb) {
+        if (kb + 1 < nkb) WAIT_VM(FEW_INST);
+        else WAIT_VM(0);
+        if (kb == 0) first();
+        LDS_BARRIER();
+        if (kb + 2 < nkb) few_issue(t, st + nxt * SB, kb + 2);
+        u32x4 wq[4], xq[4];
+        frag64(st + cur * SB, wv * 32 + c, h, wq);
+        frag64(st + cur * SB, 128 + (c & (FP8_FEW - 1)), h, xq);
+        h8 wa[8], xa[8];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            e4m3_to_h16(wq[i], wa[2 * i], wa[2 * i + 1]);
+            e4m3_to_h16(xq[i], xa[2 * i], xa[2 * i + 1]);
+        }
+        block_acc16(xa, wa, scl[kb], acc);
+    };
+    few_issue(t, st, 0);
+    if (nkb > 1) few_issue(t, st + SB, 1);
+    for (int kb = 0; kb < nkb; kb += 3) {
+        step(0, 2, kb);
+        if (kb + 1 < nkb) step(1, 0, kb + 1);
+        if (kb + 2 < nkb) step(2, 1, kb + 2);
+    }
+}
+
+// grid (N/64, segments): waves 0, 1 the gate columns, waves 2, 3 the same up columns; the up sums reach the gate waves
+// through LDS for the SwiGLU. Accumulator registers 0 .. 3 hold rows 4 (lane / 32) + r, the only ones a segment can have.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fp8_gateup_few_kernel(Fp8Args a) {
+    __shared__ __align__(16) unsigned char st[3 * FEW_ROWS * 128];
+    __shared__ float scl[2 * FP8_MAX_KB];
+    __shared__ float rsx[FP8_FEW];
+    const int cb = blockIdx.x, s = blockIdx.y;
+    if (s >= a.nseg[0]) return;
+    const int e = a.seg_expert[s], row0 = a.seg_row0[s], rn = a.seg_rows[s];
+    if (rn <= 0) return;                                             // (no rows: nothing to stage or store)
+    const int lane = threadIdx.x & 63, ti = threadIdx.x;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int K = a.K, N = a.N, nkb = K >> 7;
+    const int tk = a.tok[row0 + min(lane >> 3, rn - 1)];             // the activation row this lane stages
+    FewTile t;
+#pragma unroll
+    for (int j = 0; j < FEW_INST; ++j) {
+        const int R = j < FEW_INST - 1 ? wv * 32 + j * 8 + (lane >> 3) : 128 + (lane >> 3);
+        const uint8_t* rowp = R < 64    ? a.w13 + ((size_t)e * 2 * N + cb * 64 + R) * K
+                              : R < 128 ? a.w13 + ((size_t)e * 2 * N + N + cb * 64 + (R - 64)) * K
+                                        : a.qx + (size_t)tk * K;
+        t.src[j] = rowp + (((lane & 7) ^ swz(R)) << 4);
+        t.lds[j] = (j < FEW_INST - 1 ? wv * 32 + j * 8 : 128) * 128;
+    }
+    const int tsc = min(ti, 2 * nkb - 1);
+    const float scv = a.w13s[((size_t)e * (2 * N / 128) + (tsc < nkb ? 0 : N / 128) + cb / 2) * nkb +
+                             (tsc < nkb ? tsc : tsc - nkb)];
+    const float sxv = a.sx[a.tok[row0 + min(ti & (FP8_FEW - 1), rn - 1)]];
+    f32x16 acc = {};
+    few_gemm(t, st, nkb, wv, lane, scl + (wv >> 1) * nkb, [&]() {
+        if (ti < 2 * nkb) scl[ti] = scv;
+        if (ti < FP8_FEW) rsx[ti] = sxv;
+    }, acc);
+    __syncthreads();                                                 // the stages are no longer read
+    float4* ex = reinterpret_cast<float4*>(st);                      // [2][64] up sums (rows 0 .. 3 of the lane)
+    if (wv >= 2) ex[(wv - 2) * 64 + lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    __syncthreads();
+    if (wv >= 2) return;
+    const float4 u4 = ex[wv * 64 + lane];
+    const float uu[4] = {u4.x, u4.y, u4.z, u4.w};
+    const float L = a.limit;
+    const int col = cb * 64 + wv * 32 + (lane & 31);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int row = 4 * (lane >> 5) + r;
+        const float sx = rsx[min(row, rn - 1)];
+        float gv = acc[r] * sx, uv = uu[r] * sx;
+        if (L != 0.0f) {
+            gv = fminf(gv, L);
+            uv = fminf(fmaxf(uv, -L), L);
+        }
+        const float act = __fdiv_rn(gv, 1.0f + (float)exp(-(double)gv)) * uv;
+        if (row < rn) a.a16[(size_t)(row0 + row) * N + col] = (uint16_t)h_as_u16((_Float16)act);
+    }
+}
+
+// grid (K/128, segments): wave w owns columns 32 w .. + 31 of the block.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void fp8_down_few_kernel(Fp8Args a) {
+    __shared__ __align__(16) unsigned char st[3 * FEW_ROWS * 128];
+    __shared__ float scl[FP8_MAX_KB];
+    const int cb = blockIdx.x, s = blockIdx.y;
+    if (s >= a.nseg[0]) return;
+    const int e = a.seg_expert[s], row0 = a.seg_row0[s], rn = a.seg_rows[s];
+    if (rn <= 0) return;                                             // (no rows: nothing to stage or store)
+    const int lane = threadIdx.x & 63, ti = threadIdx.x;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int K = a.K, N = a.N, nkb = N >> 7;
+    FewTile t;
+#pragma unroll
+    for (int j = 0; j < FEW_INST; ++j) {
+        const int R = j < FEW_INST - 1 ? wv * 32 + j * 8 + (lane >> 3) : 128 + (lane >> 3);
+        const uint8_t* rowp = R < 128 ? a.w2 + ((size_t)e * K + cb * 128 + R) * N
+                                      : a.qa + (size_t)(row0 + min(R - 128, rn - 1)) * N;
+        t.src[j] = rowp + (((lane & 7) ^ swz(R)) << 4);
+        t.lds[j] = (j < FEW_INST - 1 ? wv * 32 + j * 8 : 128) * 128;
+    }
+    const float scv = a.w2s[((size_t)e * (K / 128) + cb) * nkb + min(ti, nkb - 1)];
+    float sa[4], rw[4];
+    int pe[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {                                    // this lane's rows (loaded ahead of the stages)
+        const int pos = row0 + min(4 * (lane >> 5) + r, rn - 1);
+        sa[r] = a.sa[pos];
+        rw[r] = a.w32[pos];
+        pe[r] = a.pe[pos];
+    }
+    f32x16 acc = {};
+    few_gemm(t, st, nkb, wv, lane, scl, [&]() {
+        if (ti < nkb) scl[ti] = scv;
+    }, acc);
+    const int col = cb * 128 + wv * 32 + (lane & 31);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int row = 4 * (lane >> 5) + r;
+        if (row < rn && pe[r] >= 0) a.contrib[(size_t)(row0 + row) * K + col] = rw[r] * (acc[r] * sa[r]);
+    }
+}
+
 // grid (ceil(T/4), K/256), 256 threads: one wave per (token t, 256 columns), 4 columns per lane. out[t] = sum over
 // the token's slots k (in order) of the valid pairs' contributions, converted to the output dtype (deterministic:
 // no atomics).
@@ -471,10 +619,13 @@ int launch_quant_rows(const void* x, int xdt, int64_t stride, int rows, int K, u
 int launch_fp8(const Fp8Args& a, hipStream_t st, int kernels) {
     if (kernels & 1)
         quant_rows(a.x, a.xdt, a.x_stride, a.T, a.K, a.qx, a.sx, st);
-    if (kernels & 2) hipLaunchKernelGGL(fp8_gateup_kernel, dim3(a.N / 64, a.S_cap), dim3(256), 0, st, a);
+    const bool few = fp8_seg_rows(a.T) == FP8_FEW;
+    if ((kernels & 2) && few) hipLaunchKernelGGL(fp8_gateup_few_kernel, dim3(a.N / 64, a.S_cap), dim3(256), 0, st, a);
+    else if (kernels & 2) hipLaunchKernelGGL(fp8_gateup_kernel, dim3(a.N / 64, a.S_cap), dim3(256), 0, st, a);
     if (kernels & 4) {
         quant_rows(a.a16, DT_F16, a.N, a.P, a.N, a.qa, a.sa, st);
-        hipLaunchKernelGGL(fp8_down_kernel, dim3(a.K / 128, a.S_cap), dim3(256), 0, st, a);
+        if (few) hipLaunchKernelGGL(fp8_down_few_kernel, dim3(a.K / 128, a.S_cap), dim3(256), 0, st, a);
+        else hipLaunchKernelGGL(fp8_down_kernel, dim3(a.K / 128, a.S_cap), dim3(256), 0, st, a);
     }
     if (kernels & 8) hipLaunchKernelGGL(fp8_combine_kernel, dim3((a.T + 3) / 4, a.K / 256), dim3(256), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;

@@ -287,6 +287,12 @@ struct Fp8Args {
     int64_t out_stride;
 };
 constexpr int FP8_TM = 64;   // rows per segment (two 32-row MFMA tiles)
+// Calls of up to FP8_FEW_T tokens take segments of FP8_FEW rows and kernels that stage only those: 17 instead of 24 KB per
+// stage, so three workgroups (96 KB of weights in flight) share a CU instead of two (64 KB). An expert with more rows is
+// read once per segment, at most twice here.
+// T = 12, 288 experts, hidden 4096, intermediate 1024: 235 -> 188 us.
+constexpr int FP8_FEW = 8, FP8_FEW_T = 16;
+constexpr int fp8_seg_rows(int64_t tokens) { return tokens <= FP8_FEW_T ? FP8_FEW : FP8_TM; }
 // kernels: bit 0 quantize inputs, bit 1 gate/up, bit 2 down-input quantization + down, bit 3 slot-order combine
 int launch_fp8(const Fp8Args& a, hipStream_t st, int kernels);
 int launch_quant_rows(const void* x, int xdt, int64_t stride, int rows, int K, uint8_t* q, float* s, hipStream_t st);

@@ -133,3 +133,26 @@ def test_full_configuration_token_sample(cuda):
     assert np.allclose(torch.from_numpy(got).to(torch.bfloat16).float().numpy(), ref, rtol=2e-2, atol=1e-3)
     assert _rel(got, ref64) <= 5e-3, _rel(got, ref64)
     assert np.isfinite(out.cpu().numpy()).all()
+
+
+@pytest.mark.parametrize("K,N", [(256, 128), (512, 384), (4096, 256)])
+@pytest.mark.parametrize("T", [1, 7, 8, 9, 16])
+def test_few_tokens(cuda, K, N, T):
+    """Calls of up to 16 tokens run on segments of at most 8 rows: each token's output equals its output in a call of 40
+    tokens on the 64-row kernels bit for bit, and the oracle's to rel_l2 <= 1e-6. Expert 0 takes every token (one segment,
+    or two from 9 tokens)."""
+    from mi355moe import fp8, synthetic
+    print(f"fp8 few T={T} K={K} N={N}", flush=True)
+    n, topk = 6, 3
+    ex = synthetic.fp8_layer(n, K, N, seed=31, device="cuda")
+    x = synthetic.activations(40, K, seed=32, device="cuda")
+    ids, w = _routing(40, n, topk, seed=33)
+    ids[:, 0], ids[:, 1:] = 0, 1 + ids[:, 1:] % (n - 1)
+    ids[ids[:, 1] == ids[:, 2], 2] = -1
+    run = lambda t: fp8.moe_forward_ids(ex, x[:t], torch.from_numpy(ids[:t]).cuda(), torch.from_numpy(w[:t]).cuda(),
+                                        limit=10.0, out_dtype=torch.float32)
+    got = run(T)
+    assert torch.equal(got, run(40)[:T])
+    tok, exs, pw = e4m3.pairs_fp32(ids[:T], w[:T], n)
+    ref = e4m3.forward(_host_layer(ex), x[:T].float().cpu().numpy(), tok, exs, pw, 10.0, "kernel")
+    assert _rel(got.cpu().numpy(), ref) <= 1e-6
