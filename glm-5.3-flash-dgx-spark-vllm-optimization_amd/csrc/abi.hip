@@ -1,5 +1,6 @@
 // C-ABI entry points: argument checks (all before the first launch), launch planning and workspace layout.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -76,31 +77,50 @@ int pow2ceil(int64_t v) {
     return p;
 }
 
-DecodePlan plan_decode(int64_t P, int64_t rows_bound, int64_t n, int64_t K, int64_t N, int shared_suh) {
+// Experts of n that T tokens of topk distinct picks among total ids reach, for uniform routing.
+double expected_experts(int64_t T, int64_t topk, int64_t n, int64_t total) {
+    return (double)n * (1.0 - std::pow(1.0 - std::min(1.0, (double)topk / (double)total), (double)T));
+}
+
+// Splits of a reduction whose unsplit grid has w workgroups: the fewest that give more workgroups than half the CUs. One
+// split needs no cross-workgroup reduction, and a second workgroup on a CU gains little (one already keeps its VALU
+// nearly busy), so filling both slots of every CU (a target of 400) loses more to the partial sums than it gains. Layer
+// call at 288 experts, hidden 4096, target 129 against 400 (and 257): intermediate 1024 T = 1 38.0 / 43.6 (42) us, 2
+// 46.3 / 53.0 (50), 3 59.8 / 77.8 (64); intermediate 512 T = 1 35.1 / 41.6, 3 42.9 / 58.7; intermediate 256 T = 3
+// 34.3 / 49.5, 6 44.2 / 58.4 (47), 12 64.2 / 69.0. A grid
+// that fills the CUs and 5 to 29 % of a second round is split once more (intermediate 1024, w = 302, T = 5: 96.8 against
+// 103.7 us; 297, 144 experts, top-6: 90.7 / 99.1), for up to 64 pairs; not a fuller one (w = 358: 114 / 104) nor one that
+// just fits (259: 70 / 65).
+int64_t splits_for(double w, int64_t P) {
+    int64_t c = 1;
+    while (w * (double)c < 129.0 && c < 16) c *= 2;
+    if (P <= 64 && w * (double)c > 270.0 && w * (double)c <= 330.0) c *= 2;
+    return c;
+}
+
+// topk > 0: the pairs are T x topk distinct picks; 0: any pairs.
+DecodePlan plan_decode(int64_t P, int64_t rows_bound, int64_t n, int64_t K, int64_t N, int shared_suh, int64_t topk) {
     DecodePlan d;
     d.rmax = (int)std::min<int64_t>(16, pow2ceil(std::max<int64_t>(1, rows_bound)));
     d.seg = d.rmax;
     d.S_cap = (int)(std::min(P, n) + (P + d.seg - 1) / d.seg);
-    const int64_t s_est = std::max<int64_t>(1, std::min(P, n));
-    // Splits of the reduction: the fewest that give more workgroups than half the CUs, whose staged input rows fit
-    // DECODE_LDS_MAX in some number of passes. One split needs no cross-workgroup reduction, and a second workgroup on
-    // a CU gains little (one already keeps its VALU nearly busy), so filling both slots of every CU (a target of 400)
-    // loses more to the partial sums than it gains. Layer call at 288 experts, hidden 4096, target 129 against 400 (and
-    // 257): intermediate 1024 T = 1 38.0 / 43.6 (42) us, 2 46.3 / 53.0 (50), 3 59.8 / 77.8 (64); intermediate 512
-    // T = 1 35.1 / 41.6, 3 42.9 / 58.7; intermediate 256 T = 3 34.3 / 49.5, 6 44.2 / 58.4 (47), 12 64.2 / 69.0.
-    const int64_t target = 129;
+    const double s_est = topk > 0 ? std::max(1.0, expected_experts(P / topk, topk, n, n))
+                                  : (double)std::max<int64_t>(1, std::min(P, n));
+    // whose staged input rows fit DECODE_LDS_MAX in some number of passes
+    const int64_t want_gu = splits_for(s_est * (double)(N / 128), P);
     int64_t sk = 0;
     for (int64_t c : {1, 2, 4, 8, 16}) {
         if (K % c || (K / c) % 256 || !decode_lds_gateup(d.rmax, (int)(K / c), shared_suh)) continue;
         sk = c;
-        if (s_est * (N / 128) * c >= target) break;
+        if (c >= want_gu) break;
     }
     d.sk_gu = (int)std::max<int64_t>(1, sk);
+    const int64_t want_dn = splits_for(s_est * (double)((K + 511) / 512), P);   // 512-column down workgroups
     int64_t nr = N;
     for (int64_t c : {1, 2, 4, 8}) {
         if (N % c || (N / c) % 128 || decode_lds_down(d.rmax, (int)(N / c)) > DECODE_LDS_MAX) continue;
         nr = N / c;
-        if (s_est * ((K + 511) / 512) * c >= target) break;   // 512-column down workgroups
+        if (c >= want_dn) break;
     }
     d.sk_dn = (int)(N / nr);
     d.kch_gu = (int)(K / d.sk_gu);
@@ -493,7 +513,7 @@ int64_t mi355moe_moe_workspace_bytes_path(const mi355moe_exl3_layer* layer, int6
         return (int64_t)w.bytes;
     }
     const DecodePlan p = plan_decode(P, std::max<int64_t>(1, T), layer->n, layer->hidden, layer->intermediate,
-                                     shared_flag(layer));
+                                     shared_flag(layer), topk);
     DecodeWs w;
     carve_decode(nullptr, P, layer->n, layer->hidden, layer->intermediate, p, true, w);
     return (int64_t)w.bytes;
@@ -531,12 +551,28 @@ int mi355moe_moe_forward_ids(const mi355moe_exl3_layer* layer, const void* x, in
 // sets the id and weight sources).
 static int prep_decode(const mi355moe_exl3_layer* layer, const void* x, int x_dtype, int64_t x_stride, int64_t T,
                        int64_t topk, float limit, void* out, int out_dtype, int64_t out_stride, void* workspace,
-                       size_t workspace_bytes, DecodePlan& p, DecodeWs& w) {
+                       size_t workspace_bytes, int64_t n_global, DecodePlan& p, DecodeWs& w) {
     const int64_t K = layer->hidden, N = layer->intermediate, n = layer->n, P = T * topk;
-    p = plan_decode(P, T, n, K, N, shared_flag(layer));
+    p = plan_decode(P, T, n, K, N, shared_flag(layer), topk);
     if (p.S_cap > 65535) return MI355MOE_ELIMIT;
     carve_decode(workspace, P, n, K, N, p, true, w);
     if (workspace_bytes < w.bytes) return MI355MOE_EWORKSPACE;
+    if (n_global > n && T > 0) {
+        // an expert-parallel rank reaches fewer of its experts than the plan (and the workspace query, which does not
+        // know the map) assumes: gate/up splits for those, where their partial sums fit the contribution buffer, which
+        // is free until the down kernel (hidden 4096, top-8, split / not: 96 of 192 experts, intermediate 256, T = 15
+        // 45.5 / 54.0 us, 24 47.4 / 55.6; 144 of 288, intermediate 512, T = 6 42.7 / 51.9, intermediate 256, T = 8
+        // 35.4 / 39.1)
+        int64_t c = splits_for(std::max(1.0, expected_experts(T, topk, n, n_global)) * (double)(N / 128), P);
+        while (c > p.sk_gu && (K % c || (K / c) % 256 || 2 * c * N > K ||
+                               !decode_lds_gateup(p.rmax, (int)(K / c), shared_flag(layer))))
+            c /= 2;
+        if (c > p.sk_gu) {
+            p.sk_gu = (int)c;
+            p.kch_gu = (int)(K / c);
+            w.da.zg = w.da.contrib;
+        }
+    }
     RouteArgs& r = w.ra;
     r.P = (int)P;
     r.topk = (int)topk;
@@ -711,7 +747,7 @@ int mi355moe_moe_forward_ids_opt(const mi355moe_exl3_layer* layer, const void* x
     DecodePlan p;
     DecodeWs w;
     if (int rc = prep_decode(layer, x, x_dtype, x_stride, T, topk, limit, out, out_dtype, out_stride, workspace,
-                             workspace_bytes, p, w))
+                             workspace_bytes, expert_map ? n_global : 0, p, w))
         return rc;
     RouteArgs& r = w.ra;
     r.ids = ids;
@@ -749,7 +785,7 @@ void carve_split(void* ws, int64_t P, int64_t T, int64_t n, int64_t K, int64_t N
     memset(&w.da, 0, sizeof(w.da));
     memset(&w.pa, 0, sizeof(w.pa));
     DecodePlan& p = w.dp;
-    p = plan_decode(P, std::max<int64_t>(1, cap), n, K, N, shared);
+    p = plan_decode(P, std::max<int64_t>(1, cap), n, K, N, shared, 0);
     p.S_cap = (int)std::min<int64_t>(p.S_cap, n * ((std::max<int64_t>(1, cap) + p.seg - 1) / p.seg));
     const int S_fat = (int)(std::min(P, n) + (P + PREFILL_TM - 1) / PREFILL_TM);
     RouteArgs& r = w.thin;
@@ -1002,7 +1038,7 @@ int mi355moe_moe_layer(const mi355moe_exl3_layer* layer, const void* x, int x_dt
         DecodePlan p;
         DecodeWs w;
         if (int rc = prep_decode(layer, x, x_dtype, x_stride, T, topk, limit, out, out_dtype, out_stride, workspace,
-                                 (size_t)base, p, w))
+                                 (size_t)base, 0, p, w))
             return rc;
         RouteArgs& r = w.ra;
         r.ids = ids;
@@ -1561,7 +1597,7 @@ int64_t mi355moe_exl3_moe_workspace_bytes(const mi355moe_exl3_layer* layer, int6
     size_t most = 0;                                  // the plan depends on the row cap: take the largest layout
     for (int64_t rows = 1; rows <= 16; rows *= 2) {
         const DecodePlan p = plan_decode(Pp, std::min(Pp, rows), layer->n, layer->hidden, layer->intermediate,
-                                         shared_flag(layer));
+                                         shared_flag(layer), 0);
         DecodeWs w;
         carve_decode(nullptr, Pp, layer->n, layer->hidden, layer->intermediate, p, false, w);
         most = std::max(most, w.bytes);
@@ -1583,7 +1619,7 @@ int mi355moe_exl3_moe(const mi355moe_exl3_layer* layer, const void* hidden, int6
     if (P < 0 || P > MAX_PAIRS) return MI355MOE_ELIMIT;
     if (P == 0) return 0;
     const int64_t K = layer->hidden, N = layer->intermediate, n = layer->n;
-    const DecodePlan p = plan_decode(P, std::min(P, max_rows), n, K, N, shared_flag(layer));
+    const DecodePlan p = plan_decode(P, std::min(P, max_rows), n, K, N, shared_flag(layer), 0);
     if (p.S_cap > 65535) return MI355MOE_ELIMIT;
     DecodeWs w;
     carve_decode(workspace, P, n, K, N, p, false, w);

@@ -36,3 +36,26 @@ def test_rank(cuda, monkeypatch, T, topk, local):
                                          w.cpu().numpy(), local, topk)
     ref = moe.forward(lay, x.cpu().to(torch.float16).numpy(), tok, e, w16, 10.0, "e3")
     assert np.linalg.norm(got["auto"] - ref) <= 5e-4 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("T", [1, 8, 15])
+def test_rank_decode(cuda, T):
+    """Decode calls of a rank with 96 of 192 experts: the gate/up reduction splits for the experts the rank reaches, its
+    partial sums in the contribution buffer."""
+    from mi355moe import _lib, ops, synthetic
+    n, n_global, K, N, topk = 96, 192, 4096, 256, 8
+    print(f"ep rank decode T={T}", flush=True)
+    ex = synthetic.calibrated_layer(n, K, N, seed=25, device=cuda, uniform_suh=True)
+    x = synthetic.activations(T, K, seed=26, device=cuda)
+    ids = torch.rand(T, n_global, generator=torch.Generator().manual_seed(27)).topk(topk, 1).indices.to(torch.int32).to(cuda)
+    w = synthetic.softmax_weights(T, topk, seed=28, device=cuda)
+    emap = torch.full((n_global,), -1, dtype=torch.int64)
+    emap[::2] = torch.arange(n)
+    got = ops.moe_forward_ids(ex, x, ids, w, out_dtype=torch.float32, expert_map=emap.to(cuda),
+                              path=_lib.PATH_DECODE).cpu().numpy()
+    lay = {k: getattr(ex, k).cpu().numpy() for k in ("w13_trellis", "w13_suh", "w13_svh", "w2_trellis", "w2_suh",
+                                                     "w2_svh")}
+    tok, e, w16 = moe.pairs_from_routing(routing.map_topk_to_local(ids.cpu().numpy(), n, emap.numpy()),
+                                         w.cpu().numpy(), n, topk)
+    ref = moe.forward(lay, x.cpu().to(torch.float16).numpy(), tok, e, w16, 10.0, "decode_x")
+    assert np.linalg.norm(got - ref) <= 5e-4 * np.linalg.norm(ref)
