@@ -54,6 +54,12 @@ int tok_rows_flag(const mi355moe_exl3_layer* L) {
     return (L->flags & MI355MOE_LAYER_SHARED_W13_SUH) && (L->flags & MI355MOE_LAYER_UNIFORM_W13_SUH) ? 1 : 0;
 }
 
+// The same for the grouped GEMMs, whose staging addresses token rows by 32-bit byte offsets: larger row buffers keep one
+// row per pair (addressed from the segment's first row).
+int grouped_tok_rows(const mi355moe_exl3_layer* L, int64_t T) {
+    return tok_rows_flag(L) && T * L->hidden * 2 < (int64_t(1) << 32) ? 1 : 0;
+}
+
 // Pairs of P expected on n local experts: with an expert map over more global ids, their share of the ids.
 int64_t local_pairs(int64_t P, int64_t n, const int64_t* expert_map, int64_t n_global) {
     return expert_map && n_global > n ? std::max<int64_t>(1, P * n / n_global) : P;
@@ -669,7 +675,7 @@ static int run_grouped(const mi355moe_exl3_layer* layer, const void* x, int x_dt
     d.odt = dt_w(out_dtype);
     d.out_stride = out_stride;
     d.e4m3 = e4m3 ? 1 : 0;
-    d.tok_rows = tok_rows_flag(layer);
+    d.tok_rows = grouped_tok_rows(layer, T);
     d.pairs_local = (int)local_pairs(P, n, expert_map, n_global);
     d.contrib_bf16 = (options & MI355MOE_OPT_BF16_CONTRIB) ? 1 : 0;
     d.out_accumulate = (options & MI355MOE_OPT_ACCUMULATE) ? 1 : 0;
@@ -924,7 +930,7 @@ int mi355moe_moe_forward_ids_split(const mi355moe_exl3_layer* layer, const void*
     a.xdt = dt_act(x_dtype);
     a.x_stride = x_stride;
     a.tok = w.fat.tok;
-    a.tok_rows = tok_rows_flag(layer);
+    a.tok_rows = grouped_tok_rows(layer, T);
     a.pairs_local = (int)local_pairs(P, n, expert_map, n_global);
     a.w16 = w.fat.w16;
     a.pe = w.fat.pe;
