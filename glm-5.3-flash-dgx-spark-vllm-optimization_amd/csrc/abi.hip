@@ -54,10 +54,11 @@ int tok_rows_flag(const mi355moe_exl3_layer* L) {
     return (L->flags & MI355MOE_LAYER_SHARED_W13_SUH) && (L->flags & MI355MOE_LAYER_UNIFORM_W13_SUH) ? 1 : 0;
 }
 
-// The same for the grouped GEMMs, whose staging addresses token rows by 32-bit byte offsets: larger row buffers keep one
-// row per pair (addressed from the segment's first row).
+// The grouped GEMMs address token rows by 32-bit byte offsets (pf_gemm): a buffer of more bytes holds one row per pair
+// instead, addressed from the segment's first row. Every place that sets PrefillArgs::tok_rows for a GEMM asks here.
+bool tok_rows_fit(int64_t tokens, int64_t K) { return tokens * K * 2 < (int64_t(1) << 32); }
 int grouped_tok_rows(const mi355moe_exl3_layer* L, int64_t T) {
-    return tok_rows_flag(L) && T * L->hidden * 2 < (int64_t(1) << 32) ? 1 : 0;
+    return tok_rows_flag(L) && tok_rows_fit(T, L->hidden) ? 1 : 0;
 }
 
 // Pairs of P expected on n local experts: with an expert map over more global ids, their share of the ids.
@@ -675,7 +676,7 @@ static int run_grouped(const mi355moe_exl3_layer* layer, const void* x, int x_dt
     d.odt = dt_w(out_dtype);
     d.out_stride = out_stride;
     d.e4m3 = e4m3 ? 1 : 0;
-    d.tok_rows = grouped_tok_rows(layer, T);
+    d.tok_rows = d.tok_scales = grouped_tok_rows(layer, T);
     d.pairs_local = (int)local_pairs(P, n, expert_map, n_global);
     d.contrib_bf16 = (options & MI355MOE_OPT_BF16_CONTRIB) ? 1 : 0;
     d.out_accumulate = (options & MI355MOE_OPT_ACCUMULATE) ? 1 : 0;
@@ -1485,8 +1486,12 @@ int mi355moe_e4m3_fused(const uint8_t* a8, const float* asc, int64_t a8_rows, ui
     a.out = out;
     a.odt = dt_w(out_dtype);
     a.out_stride = out_stride;
-    if (tok_rows) {                                   // row r's gate/up input is a8 row row_token[r]
-        a.tok_rows = 1;
+    // TOKEN_ROWS: row r's gate/up input is a8 row row_token[r]. The token rows are widened once each, or, where they
+    // would not fit the GEMM's offsets, the routed rows are (into the same buffer)
+    const bool widen_tok = tok_rows && tok_rows_fit(tokens, K);
+    if (tok_rows) {
+        a.tok_rows = widen_tok ? 1 : 0;
+        a.tok_scales = 1;
         a.tok = w.tok32;
     }
     RowsPlan rp;
@@ -1498,9 +1503,10 @@ int mi355moe_e4m3_fused(const uint8_t* a8, const float* asc, int64_t a8_rows, ui
     rp.list = w.list;
     rp.tok32 = tok_rows ? w.tok32 : nullptr;
     rp.a8 = a8;
-    rp.a8_rows = (int)(tok_rows ? tokens : rows_cap);
+    rp.a8_rows = (int)(widen_tok ? tokens : rows_cap);
     rp.a8_cols = (int)K;
-    rp.a8_all = tok_rows ? 1 : 0;
+    rp.a8_all = widen_tok ? 1 : 0;
+    rp.a8_tok = tok_rows && !widen_tok ? 1 : 0;
     rp.a8_dst = w.h13;
     rp.kernels = 2 | 4;
     if (seg_cap <= rows_cap) {                        // the one-launch schedule where the tile choice takes it

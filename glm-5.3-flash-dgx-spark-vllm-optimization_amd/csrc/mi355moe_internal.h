@@ -153,8 +153,9 @@ struct PrefillArgs {
     // thin/fat split: rows with pe < 0 and pe_thin >= 0 were computed by the decode kernels, whose contrib rows hold
     // finished contributions (the combine adds them as they are); nullptr: no split
     const int* pe_thin;
-    // every expert shares one w13 suh: h13 (and, e4m3, asc) hold one row per token, row pos reads token tok[pos]'s
-    int tok_rows;
+    // every expert shares one w13 suh: h13 holds one row per token (below 4 GiB in all, the GEMM's offsets are 32-bit),
+    // row pos reads token tok[pos]'s; tok_scales: the same for the e4m3 activation scales asc
+    int tok_rows, tok_scales;
     int contrib_bf16;       // the down kernel stores its raw accumulators as bf16 (contrib viewed as bf16 [P][K])
     int out_accumulate;     // the combine adds the routed sum to out's current values (the shared-expert fold)
     int small_rows;         // > 0: segments of at most this many rows go to the small-tile GEMMs, larger ones to the
@@ -233,7 +234,7 @@ int launch_prefill(const PrefillArgs& a, hipStream_t st, int kernels);
 // A call over caller-built row tables (rows a.P = rows_cap, segments a.seg_* / a.nseg, chunk a.chunk / a.nchunks):
 // the rows the live segments cover are marked in pe (their segment's expert, or a.row_expert[r]), every other row -1;
 // then optionally e4m3 code rows widened into the GEMMs' fp16 staging (a8 -> a8_dst: every row < a8_rows, or only the
-// marked ones), launch_prefill's `kernels` over the marked rows, and with tokens > 0 every token's marked rows
+// marked ones, with a8_tok row r from a8 row tok32[r]), launch_prefill's `kernels` over the marked rows, and with tokens > 0 every token's marked rows
 // (row_token) summed in row order and ADDED to out (fp32 or bf16 [tokens][K], row stride a.out_stride) with the row
 // weights a.w32 (fp32) or a.w16 (fp16). tok32 (optional): [P] the rows' tokens as int32 (outside [0, tokens): 0), for
 // token-row A operands. cnt [tokens], list [tokens][PF_ROWS_PER_TOKEN] and pe [P] are scratch.
@@ -245,7 +246,7 @@ struct RowsPlan {
     int2* list;
     int* tok32;
     const uint8_t* a8;
-    int a8_rows, a8_cols, a8_all;
+    int a8_rows, a8_cols, a8_all, a8_tok;
     uint16_t* a8_dst;
     int kernels;
 };

@@ -546,7 +546,7 @@ __device__ __forceinline__ void pf_gemm(const PfTile& t, unsigned char* smem, f1
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int steps = t.kdim / (16 * PF_KT);
     // A DMA sources: instruction i of this wave = rows RPW wv + RPI i + lane / CPR, slot lane % CPR (byte offsets from
-    // a_rows: below 2^32, the host keeps token-row buffers of more bytes off this path)
+    // a_rows: below 2^32, the host takes tok_rows only for buffers of fewer bytes)
     uint32_t aoff[NA];
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
@@ -810,7 +810,7 @@ __device__ __forceinline__ void pf_gateup_tile(const PrefillArgs& a, int s, int 
 #pragma unroll
             for (int p = 0; p < 2; ++p) {
                 const int ar = row0 + min(32 * rb + wv * 8 + p * 4 + rsub, rn - 1);
-                ri[rb][p] = a.tok_rows ? a.tok[ar] : ar;
+                ri[rb][p] = a.tok_scales ? a.tok[ar] : ar;
             }
 #pragma unroll
         for (int rb = 0; rb < SUB / 32; ++rb)
@@ -1449,14 +1449,16 @@ __global__ __launch_bounds__(256) void pf_seg_rows_kernel(PrefillArgs a, int* pe
 
 // e4m3 code rows (one byte per element, in the staging order of h13 / h2) widened to the fp16 staging rows the GEMMs
 // read: dst[r][k] = the fp16 of the e4m3 value src[r][k] (exact: every e4m3 value is an fp16), for every row r < rows
-// (pe == nullptr) or those with pe[r] >= 0. One wave per row, 16 codes per lane per pass; cols % 16 == 0.
+// (pe == nullptr) or those with pe[r] >= 0 (tok: from src row tok[r]). One wave per row, 16 codes per lane per pass;
+// cols % 16 == 0.
 __global__ __launch_bounds__(256) void pf_widen8_kernel(const uint8_t* __restrict__ src, uint16_t* __restrict__ dst,
-                                                        int cols, int rows, const int* __restrict__ pe) {
+                                                        int cols, int rows, const int* __restrict__ pe,
+                                                        const int* __restrict__ tok) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
     for (int r = wave; r < rows; r += gridDim.x * 4) {
         if (pe && pe[r] < 0) continue;                               // uniform: one row per wave
-        const uint8_t* sr = src + (size_t)r * cols;
+        const uint8_t* sr = src + (size_t)(tok ? tok[r] : r) * cols;
         uint16_t* dr = dst + (size_t)r * cols;
         for (int c = 16 * lane; c < cols; c += 1024) {
             const u32x4 v = *reinterpret_cast<const u32x4*>(sr + c);
@@ -1768,7 +1770,7 @@ int launch_zero_out(const PrefillArgs& a, hipStream_t st) {
 int launch_prefill_rows(const PrefillArgs& a0, const RowsPlan& p, hipStream_t st) {
     if (prefill_setup()) return -1;
     if (p.tokens > 0 && (a0.contrib_bf16 || !p.row_token || !p.cnt || !p.list)) return -1;   // fp32 accumulators
-    if (p.tok32 && !p.row_token) return -1;
+    if ((p.tok32 && !p.row_token) || (p.a8_tok && !p.tok32)) return -1;
     PrefillArgs a = a0;
     a.pe = p.pe;
     const int fill = std::max(1, std::min(2048, (std::max(a.P, p.tokens) + 255) / 256));
@@ -1777,7 +1779,8 @@ int launch_prefill_rows(const PrefillArgs& a0, const RowsPlan& p, hipStream_t st
     if (a.S_cap > 0) hipLaunchKernelGGL(pf_seg_rows_kernel, dim3(a.S_cap), dim3(256), 0, st, a, p.pe);
     if (p.a8 && p.a8_rows > 0)
         hipLaunchKernelGGL(pf_widen8_kernel, dim3(std::max(1, std::min(4096, (p.a8_rows + 3) / 4))), dim3(256), 0, st,
-                           p.a8, p.a8_dst, p.a8_cols, p.a8_rows, p.a8_all ? nullptr : p.pe);
+                           p.a8, p.a8_dst, p.a8_cols, p.a8_rows, p.a8_all ? nullptr : p.pe,
+                           p.a8_tok ? p.tok32 : nullptr);
     if (p.kernels)
         if (launch_prefill(a, st, p.kernels)) return -1;
     if (p.tokens > 0) {

@@ -378,3 +378,40 @@ def test_e4m3_ext_run(cuda, uniform, out_dtype, down16):
     else:
         assert r <= 2e-2                       # one bf16 rounding of (0.5 + contribution), steps of 2^-8 .. 2^-7
         assert np.allclose(got.float().cpu().numpy(), 0.5 + ref, rtol=2.0 ** -8, atol=2.0 ** -8)
+
+
+def test_e4m3_fused_token_rows_of_4_gib(cuda):
+    """fused() over token rows whose widened copies pass 4 GiB (tokens x K x 2 bytes; the GEMM's token-row offsets are 32
+    bits wide): the rows of the last tokens, bit-equal to the same call over per-row codes."""
+    from mi355moe import e4m3_ext, synthetic
+    K, N, n, T, rows = 4096, 128, 2, (1 << 19) + 64, 96
+    _say(f"e4m3 fused, {T} token rows of {K}")
+    ex = synthetic.calibrated_layer(n, K, N, seed=35, device=cuda, uniform_suh=True)
+    g = torch.Generator(device=cuda).manual_seed(36)
+    tokens = torch.cat([torch.arange(32), torch.arange(T - 64, T)]).to(cuda)   # wrapped, the last 64 would read the first
+    tokens = tokens[torch.randperm(rows, generator=g, device=cuda)]
+    a8 = torch.zeros(T, K, dtype=torch.uint8, device=cuda)
+    asc = torch.zeros(T, device=cuda)
+    near = torch.cat([torch.arange(64), torch.arange(T - 64, T)]).to(cuda)
+    a8[near] = torch.randint(0, 256, (128, K), generator=g, device=cuda, dtype=torch.int32).to(torch.uint8) & 0xF7
+    asc[near] = torch.rand(128, generator=g, device=cuda) * 0.01 + 0.005
+    p = ex.tables
+    i32 = dict(dtype=torch.int32, device=cuda)
+    tabs = (torch.tensor([0, 1], **i32), torch.tensor([0, 61], **i32), torch.tensor([61, 35], **i32),
+            torch.tensor([2], **i32))
+    rw = torch.rand(rows, generator=g, device=cuda) + 0.1
+    out = torch.zeros(T, K, device=cuda)
+
+    def call(codes, scales, variant):
+        a16 = torch.empty(rows, N, dtype=torch.float16, device=cuda)
+        out.zero_()
+        e4m3_ext.fused(codes, scales, None, None, a16, out, p["gate_trellis"], p["up_trellis"], p["gate_svh"],
+                       p["up_svh"], p["down_trellis"], p["down_suh"], p["down_svh"], tokens, rw, *tabs, None, 10.0,
+                       variant=variant)
+        return a16, out[tokens]
+
+    want = call(a8[tokens].contiguous(), asc[tokens].contiguous(), 0)
+    got = call(a8, asc, e4m3_ext.TOKEN_ROWS)
+    torch.cuda.synchronize()
+    assert float(want[0].abs().max()) > 0 and torch.isfinite(want[1]).all()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
