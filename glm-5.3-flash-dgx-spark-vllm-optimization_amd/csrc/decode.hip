@@ -954,20 +954,20 @@ int launch_rot_in(const void* x, int xdt, int64_t x_stride, const int* tok, cons
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-size_t decode_lds_gateup(int rmax, int kr, int shared_suh) {
-    // the largest staging of any segment of up to rmax rows that fits DECODE_LDS_MAX (0: some segment fits no pass)
+size_t decode_lds_gateup(int rmax, int kr, int shared_suh, size_t limit) {
+    // the largest staging of any segment of up to rmax rows that fits `limit` (0: some segment fits no pass)
     int staged = 0;
     for (int rn = 1; rn <= rmax; ++rn) {
-        const int b = gateup_staged(rn, kr / gateup_passes(rn, kr, shared_suh != 0, (int)DECODE_LDS_MAX), shared_suh != 0);
-        if (b > (int)DECODE_LDS_MAX) return 0;
+        const int b = gateup_staged(rn, kr / gateup_passes(rn, kr, shared_suh != 0, (int)limit), shared_suh != 0);
+        if (b > (int)limit) return 0;
         staged = std::max(staged, b);
     }
     const size_t reduce = (size_t)(4 * 64 * 16 + 2 * ZS_ROWS * 128) * 4;
     return std::max((size_t)staged, reduce);
 }
-int decode_gateup_depth(int rmax, int kr, int shared_suh) {
+static int decode_gateup_depth(int rmax, int kr, int shared_suh, int limit) {
     for (int rn = 1; rn <= rmax; ++rn)
-        if (kr / gateup_passes(rn, kr, shared_suh != 0, (int)DECODE_LDS_MAX) % 512) return 2;
+        if (kr / gateup_passes(rn, kr, shared_suh != 0, limit) % 512) return 2;
     return 4;
 }
 size_t decode_lds_down(int rmax, int kr) {
@@ -978,7 +978,7 @@ size_t decode_lds_down(int rmax, int kr) {
 template <typename F>
 static int allow_lds(F* f) {
     return hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)DECODE_LDS_MAX) == hipSuccess ? 0 : -1;
+                               (int)DECODE_LDS_ONE) == hipSuccess ? 0 : -1;
 }
 
 static int decode_setup() {
@@ -1004,10 +1004,16 @@ int launch_decode(const DecodeArgs& a0, int rmax, hipStream_t st, int kernels) {
     // load depth: four steps (of 64 k) when each wave's share of a pass holds a multiple of four, else two
     if (kernels & 1) {
         const dim3 grid(a.N / 128, a.sk_gu, a.S_cap);
-        const size_t lds = decode_lds_gateup(rmax, a.kch_gu, a.shared_suh);
-        if (lds == 0) return 1;
+        // passes halve the range, and a hidden size that is an odd multiple of 256 has no halves (nor K splits): such
+        // rows are staged whole, one workgroup per CU if need be
         a.lds_gu = (int)DECODE_LDS_MAX;                              // the passes are planned for it; lds covers them
-        const bool d4 = decode_gateup_depth(rmax, a.kch_gu, a.shared_suh) == 4;
+        size_t lds = decode_lds_gateup(rmax, a.kch_gu, a.shared_suh);
+        if (lds == 0) {
+            a.lds_gu = (int)DECODE_LDS_ONE;
+            lds = decode_lds_gateup(rmax, a.kch_gu, a.shared_suh, DECODE_LDS_ONE);
+        }
+        if (lds == 0) return 1;
+        const bool d4 = decode_gateup_depth(rmax, a.kch_gu, a.shared_suh, a.lds_gu) == 4;
         const bool multi = gateup_passes(rmax, a.kch_gu, a.shared_suh != 0, a.lds_gu) > 1;
         auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(GU_WAVES * 64), lds, st, a); };
         if (a.shared_suh && a.xrot) {

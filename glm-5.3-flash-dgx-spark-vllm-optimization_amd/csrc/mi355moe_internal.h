@@ -331,9 +331,10 @@ int launch_route_counts(const int64_t* counts64, const int64_t* token_sorted, co
 // kernels: bit 0 gate/up, bit 1 down, bit 2 combine
 int launch_decode(const DecodeArgs& a, int rmax, hipStream_t st, int kernels = 7);
 // LDS bytes of the decode GEMV workgroups staging kr reduction elements (gate/up: K range, down: N range)
-size_t decode_lds_gateup(int rmax, int kr, int shared_suh);
-size_t decode_lds_down(int rmax, int kr);
 constexpr size_t DECODE_LDS_MAX = 81920;   // two 512-thread workgroups per CU
+constexpr size_t DECODE_LDS_ONE = 163840 - 256;   // one (the whole LDS but the kernels' static words)
+size_t decode_lds_gateup(int rmax, int kr, int shared_suh, size_t limit = DECODE_LDS_MAX);
+size_t decode_lds_down(int rmax, int kr);
 int launch_rotate(const RotateArgs& a, hipStream_t st);
 int launch_dequant(const uint16_t* trellis, int kt, int nt, uint16_t* wq, hipStream_t st);
 int launch_sigmoid(const float* g, int64_t n, int variant, float* out, hipStream_t st);

@@ -40,6 +40,15 @@ def test_rows_per_segment(cuda, K, N, shared, rows):
     _check(cuda, K, N, rows, shared_suh=shared)
 
 
+# hidden sizes that are odd multiples of 256 have no halves: rows that pass the two-per-CU LDS limit are staged whole
+@pytest.mark.parametrize("K,shared,rows", [(2560, True, 16), (2816, True, 8), (2816, True, 16), (4864, True, 16),
+                                           (4864, True, 33), (1792, False, 16), (2304, False, 9)])
+def test_rows_of_odd_hidden(cuda, K, shared, rows):
+    _check(cuda, K, 128, rows, shared_suh=shared)
+    if shared:
+        _check(cuda, K, 128, rows, uniform_suh=True)
+
+
 # one w13 suh for every expert: calls of more than 4 rows rotate them once per token (with the call's first route launch,
 # or, GATEUP staged alone, in a launch of its own) and the workgroups copy them, by LDS DMA where a pass is whole 512-k pieces, by register loads where it is not or where the rows are duplicated
 @pytest.mark.parametrize("K,N", [(4096, 256), (8192, 128), (6144, 128), (768, 128), (256, 128), (10240, 128)])
