@@ -76,6 +76,7 @@ int sched_lag() {
 
 struct DecodePlan {
     int rmax, seg, S_cap, sk_gu, sk_dn, kch_gu, kch_dn;
+    int cap_gu, cap_dn;     // the most splits a call of these pairs takes (the partial-sum slots)
 };
 
 int pow2ceil(int64_t v) {
@@ -85,53 +86,81 @@ int pow2ceil(int64_t v) {
 }
 
 // Experts of n that T tokens of topk distinct picks among total ids reach, for uniform routing.
-double expected_experts(int64_t T, int64_t topk, int64_t n, int64_t total) {
-    return (double)n * (1.0 - std::pow(1.0 - std::min(1.0, (double)topk / (double)total), (double)T));
+double expected_experts(double T, int64_t topk, int64_t n, int64_t total) {
+    return (double)n * (1.0 - std::pow(1.0 - std::min(1.0, (double)topk / (double)total), T));
 }
 
-// Splits of a reduction whose unsplit grid has w workgroups: the fewest that give more workgroups than half the CUs. One
-// split needs no cross-workgroup reduction, and a second workgroup on a CU gains little (one already keeps its VALU
-// nearly busy), so filling both slots of every CU (a target of 400) loses more to the partial sums than it gains. Layer
-// call at 288 experts, hidden 4096, target 129 against 400 (and 257): intermediate 1024 T = 1 38.0 / 43.6 (42) us, 2
-// 46.3 / 53.0 (50), 3 59.8 / 77.8 (64); intermediate 512 T = 1 35.1 / 41.6, 3 42.9 / 58.7; intermediate 256 T = 3
-// 34.3 / 49.5, 6 44.2 / 58.4 (47), 12 64.2 / 69.0. A grid
-// that fills the CUs and 5 to 29 % of a second round is split once more (intermediate 1024, w = 302, T = 5: 96.8 against
-// 103.7 us; 297, 144 experts, top-6: 90.7 / 99.1), for up to 64 pairs; not a fuller one (w = 358: 114 / 104) nor one that
-// just fits (259: 70 / 65).
-int64_t splits_for(double w, int64_t P) {
-    int64_t c = 1;
-    while (w * (double)c < 129.0 && c < 16) c *= 2;
-    if (P <= 64 && w * (double)c > 270.0 && w * (double)c <= 330.0) c *= 2;
-    return c;
+// When h splits of a reduction do where more would fill both workgroup slots of every CU. A split costs partial sums, and
+// a second workgroup on a CU gains little (one keeps its VALU nearly busy), so one round of the 256 CUs is enough; but a
+// reduction split too little leaves CUs idle. wu and ws are the unsplit grid's workgroups under uniform and under skewed
+// routing, which reaches fewer experts: Zipf(1.2) routing of T tokens as many as T^0.75 uniform tokens (counted at 96 -
+// 288 experts, top-4 to -8, T = 2 - 64). Enough: the skewed grid has `keep` workgroups, and, with `tail`, the uniform one
+// does not spill up to 94 workgroups into a second round.
+// us a call by gate/up splits 1 / 2 / 4 / 8 (288 experts, hidden 4096, top-8; down unsplit), uniform and Zipf routing:
+//   intermediate 1024, T = 1: 57.7 / 48.2 / 45.0 / 49.1;  T = 5: 101 / 94 / 100 / 111, Zipf 65 / 68 / 74 / 82
+//   intermediate 512, T = 5: 62 / 66 / 66 / 73, Zipf 57 / 49 / 51 / 58
+//   intermediate 256, T = 6: 55 / 46 / 49 / 56, Zipf 56 / 46 / 43 / 46;  T = 16: 68 / 72 / 80 / 92, Zipf 64 / 57 / 56 / 64
+// and by down splits (gate/up unsplit) T = 5: intermediate 1024 101 / 99, Zipf 65 / 68; 512 62 / 63, Zipf 57 / 60: no
+// `tail` there. 3456 calls (hidden 2048 and 4096, intermediate 256 - 1024, 96 - 288 experts, top-4 to -8, T = 1 - 64,
+// each routing, half of them an expert-parallel rank of twice the experts) against the most splits, in whole calls: 2.8 %
+// faster on average, 8 of them 3 to 8 % slower; planned for uniform routing alone (129 workgroups of the local experts)
+// 510 of them were 3 to 28 % slower.
+bool splits_do(int64_t h, double wu, double ws, double keep, bool tail) {
+    constexpr double CUS = 256.0, SPILL = 350.0;
+    return ws * (double)h >= keep && !(tail && wu * (double)h > CUS && wu * (double)h <= SPILL);
 }
+constexpr double SPLIT_KEEP = 144.0;   // 9 of 16 CUs
 
-// topk > 0: the pairs are T x topk distinct picks; 0: any pairs.
-DecodePlan plan_decode(int64_t P, int64_t rows_bound, int64_t n, int64_t K, int64_t N, int shared_suh, int64_t topk) {
+// topk > 0: the pairs are T x topk distinct picks among `total` ids (fewer than n: the n local ones); topk 0: any pairs.
+// one_suh: the call rotates its rows once per token (rotate_with_route). The splits that the partial-sum buffers are laid
+// out for (cap_gu, cap_dn) depend on neither: the workspace queries do not know them.
+DecodePlan plan_decode(int64_t P, int64_t rows_bound, int64_t n, int64_t K, int64_t N, int shared_suh, int64_t topk = 0,
+                       int64_t total = 0, bool one_suh = false) {
     DecodePlan d;
     d.rmax = (int)std::min<int64_t>(16, pow2ceil(std::max<int64_t>(1, rows_bound)));
     d.seg = d.rmax;
     d.S_cap = (int)(std::min(P, n) + (P + d.seg - 1) / d.seg);
-    const double s_est = topk > 0 ? std::max(1.0, expected_experts(P / topk, topk, n, n))
-                                  : (double)std::max<int64_t>(1, std::min(P, n));
-    // whose staged input rows fit DECODE_LDS_MAX in some number of passes
-    const int64_t want_gu = splits_for(s_est * (double)(N / 128), P);
-    int64_t sk = 0;
+    const int64_t s_est = std::max<int64_t>(1, std::min(P, n)), target = 400;
+    const int64_t picks = std::max<int64_t>(1, topk), ids = std::max(total, n);
+    const double T = (double)P / (double)picks;
+    const double su = std::max(1.0, expected_experts(T, picks, n, ids));
+    const double ss = std::max(1.0, expected_experts(std::pow(T, 0.75), picks, n, ids));
+    // K splits: each half of a split spans a multiple of 128. The most: those that stage their input rows whole in
+    // DECODE_LDS_MAX and fill the slots; then fewer where that gains, with the rows staged in passes
+    auto whole = [&](int64_t c) { return decode_staged_gateup(d.rmax, (int)(K / c), shared_suh) <= DECODE_LDS_MAX; };
+    int64_t sk = 1;
     for (int64_t c : {1, 2, 4, 8, 16}) {
-        if (K % c || (K / c) % 256 || !decode_lds_gateup(d.rmax, (int)(K / c), shared_suh)) continue;
+        if (K % c || (K / c) % 256 || !whole(c)) continue;
         sk = c;
-        if (c >= want_gu) break;
+        if (s_est * (N / 128) * c >= target) break;
     }
-    d.sk_gu = (int)std::max<int64_t>(1, sk);
-    const int64_t want_dn = splits_for(s_est * (double)((K + 511) / 512), P);   // 512-column down workgroups
-    int64_t nr = N;
+    d.cap_gu = (int)sk;
+    const double wu = su * (double)(N / 128), ws = ss * (double)(N / 128);
+    while (sk > 1 && whole(sk / 2) && splits_do(sk / 2, wu, ws, SPLIT_KEEP, true)) sk /= 2;
+    // rows that need passes: unsplit and rotated once per token only (a workgroup that rotates its rows again in every
+    // pass loses up to 17 % against two whole halves), and past 4096, in passes of less than 2048, only for grids that
+    // fill the chip by themselves
+    if (sk > 1 && one_suh && !whole(1) && decode_lds_gateup(d.rmax, (int)K, shared_suh) &&
+        splits_do(1, wu, ws, K <= 4096 ? SPLIT_KEEP : 360.0, true))
+        sk = 1;
+    d.sk_gu = (int)sk;
+    const int64_t cols = (K + 511) / 512;                             // 512-column down workgroups
+    auto fits_dn = [&](int64_t c) {
+        return N % c == 0 && (N / c) % 128 == 0 && decode_lds_down(d.rmax, (int)(N / c)) <= DECODE_LDS_MAX;
+    };
+    int64_t sd = 1;
     for (int64_t c : {1, 2, 4, 8}) {
-        if (N % c || (N / c) % 128 || decode_lds_down(d.rmax, (int)(N / c)) > DECODE_LDS_MAX) continue;
-        nr = N / c;
-        if (c >= want_dn) break;
+        if (!fits_dn(c)) continue;
+        sd = c;
+        if (s_est * cols * c >= target) break;
     }
-    d.sk_dn = (int)(N / nr);
+    d.cap_dn = (int)sd;
+    while (sd > 1 && fits_dn(sd / 2) &&
+           splits_do(sd / 2, su * (double)cols, ss * (double)cols, SPLIT_KEEP, false))
+        sd /= 2;
+    d.sk_dn = (int)sd;
     d.kch_gu = (int)(K / d.sk_gu);
-    d.kch_dn = (int)nr;
+    d.kch_dn = (int)(N / d.sk_dn);
     return d;
 }
 
@@ -166,9 +195,8 @@ void carve_decode(void* ws, int64_t P, int64_t n, int64_t K, int64_t N, const De
     r.zero = reinterpret_cast<unsigned*>(d.cnt_gu);                  // both counter arrays, zeroed per call
     r.zero_words = (int64_t)((c.off - ((char*)d.cnt_gu - c.base)) / sizeof(unsigned));
     // partial-sum slots: one per chunk of a fragmented tile (none when every tile is one fragment)
-    const int64_t zs_gu = K / p.kch_gu, zs_dn = N / p.kch_dn;
-    d.zg = c.take<float>(zs_gu > 1 ? (size_t)zs_gu * 2 * P * N : 1);
-    d.zd = c.take<float>(zs_dn > 1 ? (size_t)zs_dn * P * K : 1);
+    d.zg = c.take<float>(p.cap_gu > 1 ? (size_t)p.cap_gu * 2 * P * N : 1);
+    d.zd = c.take<float>(p.cap_dn > 1 ? (size_t)p.cap_dn * P * K : 1);
     d.xd = c.take<uint16_t>((size_t)P * N);
     d.contrib = with_contrib ? c.take<float>((size_t)P * K) : nullptr;
     w.bytes = c.off;
@@ -560,26 +588,10 @@ static int prep_decode(const mi355moe_exl3_layer* layer, const void* x, int x_dt
                        int64_t topk, float limit, void* out, int out_dtype, int64_t out_stride, void* workspace,
                        size_t workspace_bytes, int64_t n_global, DecodePlan& p, DecodeWs& w) {
     const int64_t K = layer->hidden, N = layer->intermediate, n = layer->n, P = T * topk;
-    p = plan_decode(P, T, n, K, N, shared_flag(layer), topk);
+    p = plan_decode(P, T, n, K, N, shared_flag(layer), topk, n_global, tok_rows_flag(layer) != 0);
     if (p.S_cap > 65535) return MI355MOE_ELIMIT;
     carve_decode(workspace, P, n, K, N, p, true, w);
     if (workspace_bytes < w.bytes) return MI355MOE_EWORKSPACE;
-    if (n_global > n && T > 0) {
-        // an expert-parallel rank reaches fewer of its experts than the plan (and the workspace query, which does not
-        // know the map) assumes: gate/up splits for those, where their partial sums fit the contribution buffer, which
-        // is free until the down kernel (hidden 4096, top-8, split / not: 96 of 192 experts, intermediate 256, T = 15
-        // 45.5 / 54.0 us, 24 47.4 / 55.6; 144 of 288, intermediate 512, T = 6 42.7 / 51.9, intermediate 256, T = 8
-        // 35.4 / 39.1)
-        int64_t c = splits_for(std::max(1.0, expected_experts(T, topk, n, n_global)) * (double)(N / 128), P);
-        while (c > p.sk_gu && (K % c || (K / c) % 256 || 2 * c * N > K ||
-                               !decode_lds_gateup(p.rmax, (int)(K / c), shared_flag(layer))))
-            c /= 2;
-        if (c > p.sk_gu) {
-            p.sk_gu = (int)c;
-            p.kch_gu = (int)(K / c);
-            w.da.zg = w.da.contrib;
-        }
-    }
     RouteArgs& r = w.ra;
     r.P = (int)P;
     r.topk = (int)topk;
@@ -792,7 +804,7 @@ void carve_split(void* ws, int64_t P, int64_t T, int64_t n, int64_t K, int64_t N
     memset(&w.da, 0, sizeof(w.da));
     memset(&w.pa, 0, sizeof(w.pa));
     DecodePlan& p = w.dp;
-    p = plan_decode(P, std::max<int64_t>(1, cap), n, K, N, shared, 0);
+    p = plan_decode(P, std::max<int64_t>(1, cap), n, K, N, shared);
     p.S_cap = (int)std::min<int64_t>(p.S_cap, n * ((std::max<int64_t>(1, cap) + p.seg - 1) / p.seg));
     const int S_fat = (int)(std::min(P, n) + (P + PREFILL_TM - 1) / PREFILL_TM);
     RouteArgs& r = w.thin;
@@ -823,9 +835,8 @@ void carve_split(void* ws, int64_t P, int64_t T, int64_t n, int64_t K, int64_t N
     d.cnt_dn = c.take<unsigned long long>((size_t)p.S_cap * ((K + 511) / 512));
     r.zero = reinterpret_cast<unsigned*>(d.cnt_gu);
     r.zero_words = (int64_t)((c.off - ((char*)d.cnt_gu - c.base)) / sizeof(unsigned));
-    const int64_t zs_gu = K / p.kch_gu, zs_dn = N / p.kch_dn;
-    d.zg = c.take<float>(zs_gu > 1 ? (size_t)zs_gu * 2 * P * N : 1);
-    d.zd = c.take<float>(zs_dn > 1 ? (size_t)zs_dn * P * K : 1);
+    d.zg = c.take<float>(p.cap_gu > 1 ? (size_t)p.cap_gu * 2 * P * N : 1);
+    d.zd = c.take<float>(p.cap_dn > 1 ? (size_t)p.cap_dn * P * K : 1);
     d.xd = c.take<uint16_t>((size_t)P * N);
     PrefillArgs& a = w.pa;
     a.h13 = c.take<uint16_t>((size_t)P * K);
@@ -1609,7 +1620,7 @@ int64_t mi355moe_exl3_moe_workspace_bytes(const mi355moe_exl3_layer* layer, int6
     size_t most = 0;                                  // the plan depends on the row cap: take the largest layout
     for (int64_t rows = 1; rows <= 16; rows *= 2) {
         const DecodePlan p = plan_decode(Pp, std::min(Pp, rows), layer->n, layer->hidden, layer->intermediate,
-                                         shared_flag(layer), 0);
+                                         shared_flag(layer));
         DecodeWs w;
         carve_decode(nullptr, Pp, layer->n, layer->hidden, layer->intermediate, p, false, w);
         most = std::max(most, w.bytes);
@@ -1631,7 +1642,7 @@ int mi355moe_exl3_moe(const mi355moe_exl3_layer* layer, const void* hidden, int6
     if (P < 0 || P > MAX_PAIRS) return MI355MOE_ELIMIT;
     if (P == 0) return 0;
     const int64_t K = layer->hidden, N = layer->intermediate, n = layer->n;
-    const DecodePlan p = plan_decode(P, std::min(P, max_rows), n, K, N, shared_flag(layer), 0);
+    const DecodePlan p = plan_decode(P, std::min(P, max_rows), n, K, N, shared_flag(layer));
     if (p.S_cap > 65535) return MI355MOE_ELIMIT;
     DecodeWs w;
     carve_decode(workspace, P, n, K, N, p, false, w);

@@ -333,6 +333,8 @@ int launch_decode(const DecodeArgs& a, int rmax, hipStream_t st, int kernels = 7
 // LDS bytes of the decode GEMV workgroups staging kr reduction elements (gate/up: K range, down: N range)
 constexpr size_t DECODE_LDS_MAX = 81920;   // two 512-thread workgroups per CU
 constexpr size_t DECODE_LDS_ONE = 163840 - 256;   // one (the whole LDS but the kernels' static words)
+// LDS bytes of the gate/up rows staged whole, and of the kernel (in as many passes as `limit` asks; 0: they do not fit)
+size_t decode_staged_gateup(int rmax, int kr, int shared_suh);
 size_t decode_lds_gateup(int rmax, int kr, int shared_suh, size_t limit = DECODE_LDS_MAX);
 size_t decode_lds_down(int rmax, int kr);
 int launch_rotate(const RotateArgs& a, hipStream_t st);

@@ -40,8 +40,7 @@ def test_rank(cuda, monkeypatch, T, topk, local):
 
 @pytest.mark.parametrize("T", [1, 8, 15])
 def test_rank_decode(cuda, T):
-    """Decode calls of a rank with 96 of 192 experts: the gate/up reduction splits for the experts the rank reaches, its
-    partial sums in the contribution buffer."""
+    """Decode calls of a rank with 96 of 192 experts: the gate/up reduction splits for the experts the rank reaches."""
     from mi355moe import _lib, ops, synthetic
     n, n_global, K, N, topk = 96, 192, 4096, 256, 8
     print(f"ep rank decode T={T}", flush=True)
@@ -59,3 +58,29 @@ def test_rank_decode(cuda, T):
                                          w.cpu().numpy(), n, topk)
     ref = moe.forward(lay, x.cpu().to(torch.float16).numpy(), tok, e, w16, 10.0, "decode_x")
     assert np.linalg.norm(got - ref) <= 5e-4 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("T,K,N,topk", [(1, 2048, 512, 4), (3, 4096, 1024, 8), (7, 2048, 1024, 6), (24, 4096, 512, 6),
+                                        (48, 4096, 256, 8)])
+def test_rank_decode_splits(cuda, T, K, N, topk):
+    """A rank's call against one call per pick over its local ids (plans of T pairs, with other splits): the same sums in
+    another order, within the bar that each keeps to the oracle (rel_l2 <= 5e-4)."""
+    from mi355moe import _lib, ops, synthetic
+    n = 12
+    print(f"ep rank decode splits T={T} K={K} N={N} topk={topk}", flush=True)
+    ex = synthetic.calibrated_layer(n, K, N, seed=31, device=cuda, uniform_suh=True)
+    x = synthetic.activations(T, K, seed=32, device=cuda)
+    ids = torch.rand(T, 8 * n, generator=torch.Generator().manual_seed(33)).topk(topk, 1).indices.to(torch.int32)
+    ids[:, 0] = torch.arange(T, dtype=torch.int32) % n               # every token has a local expert
+    ids[:, 1:] += (ids[:, 1:] == ids[:, :1]).int() * n               # (distinct picks)
+    w = synthetic.softmax_weights(T, topk, seed=34, device=cuda)
+    emap = torch.full((8 * n + n,), -1, dtype=torch.int64)
+    emap[:n] = torch.arange(n)
+    kw = dict(out_dtype=torch.float32, path=_lib.PATH_DECODE)
+    got = ops.moe_forward_ids(ex, x, ids.to(cuda), w, expert_map=emap.to(cuda), **kw)
+    here = (ids < n).to(cuda)
+    ref = torch.zeros_like(got)
+    for k in range(topk):                                            # one pick at a time: plans of T pairs
+        one = torch.where(here[:, k:k + 1], ids[:, k:k + 1].to(cuda), -1)
+        ref += ops.moe_forward_ids(ex, x, one.int().contiguous(), w[:, k:k + 1].contiguous(), **kw)
+    assert float((got - ref).norm()) <= 5e-4 * float(ref.norm())
