@@ -199,11 +199,15 @@ constexpr int RG_MIN_T = 256;   // from this many tokens the MFMA GEMM beats the
 // loses at most 2^-23 of the chain's sum of |products|, so a chain (4 MFMAs of 16 products or 2 of 32, with their
 // accumulators at most 68 addends) is off by 68 * 2^-23 of it, and each of the K / 64 + 8 further additions by 2^-24 of
 // the whole: together (136 + K / 64 + 8) 2^-24 * sum of |x_k w_k|, itself at most |x| |w| (Cauchy-Schwarz; the norms
-// come from the same operands, 1 % added for their own rounding). T = 8192 tokens x 288 experts x 4096: bounds 63 us and
-// lazy top-k 37 us, against 525 us for every logit on the float64 matrix cores (37 TFLOP/s of 78) and 14 us for its
-// top-k; T = 64: 11 + 14 us, against 72 us for the one-launch front end.
-// Stored words: low half zero = the logit (a bf16 value); low half one = the high half is an upper bound (NaN where
-// nothing is known: sums or norms that overflow, underflow or are not finite).
+// come from the same operands, 1 % added for their own rounding). That loss is assumed of the matrix core, with room:
+// chains of cancelling, of widely spread and of one large and many small products were off by at most 5.2 of those 68
+// units in either instruction. T = 8192 tokens x 288 experts x 4096: bounds 63 us and lazy top-k 37 us, against 525 us
+// for every logit on the float64 matrix cores (37 TFLOP/s of 78) and 14 us for its top-k; T = 64: 11 + 14 us, against
+// 72 us for the one-launch front end.
+// Stored words: low half zero = the logit (a bf16 value, or 0 for one so small that its score is 0.5 all the same); low
+// half one = the high half is an upper bound. Rows whose norms do not bound anything (not finite, or past 1e37) get
+// their exact logits from the bound kernels themselves (exact_block): the top-k takes its exact dot products one after
+// another, which a token with nothing but unknown logits would pay E times.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -215,14 +219,61 @@ __device__ __forceinline__ float sum_sq8(const u32x4& v, float s) {
     }
     return s;
 }
-// The stored word of a logit from its fp32 sum s and the operands' squared norms.
+__device__ __forceinline__ bool norm_unknown(float n2) { return !(n2 < 1e37f); }
+// The stored word of a logit from its fp32 sum s and the operands' squared norms (both known). Squares below the fp32
+// range may be lost from the norms and products from the sum (up to 2^-125 each, K <= 8192): norms that this could
+// matter to bound the logit by themselves. |logit| <= 2^-26: its score rounds to 0.5, as that of 0 does.
 __device__ __forceinline__ float bound_word(float s, float x2, float w2, int K) {
+    const bool low = x2 <= 1e-25f || w2 <= 1e-25f;
+    const float xw = __builtin_sqrtf(x2 + 1e-33f) * __builtin_sqrtf(w2 + 1e-33f);
     const float c = 1.01f * (float)(144 + (K >> 6)) * 5.9604645e-8f;
-    const float d = c * __builtin_sqrtf(x2) * __builtin_sqrtf(w2) + 4.8e-7f * fabsf(s);
-    const uint32_t lo = f32_to_bf16(s - d), hi = f32_to_bf16(s + d);
-    // norms whose squares lie outside the range where fp32 sums of them hold: nothing is known
-    const bool ok = x2 > 1e-25f && x2 < 1e25f && w2 > 1e-25f && w2 < 1e25f && fabsf(s) < 1e30f;
-    return __builtin_bit_cast(float, !ok ? 0x7FFF0001u : lo == hi ? lo << 16 : (hi << 16) | 1u);
+    const float m = low ? 0.f : s, d = low ? 1.01f * xw : c * xw + 4.8e-7f * fabsf(s);
+    const uint32_t lo = f32_to_bf16(m - d), hi = f32_to_bf16(m + d);
+    const uint32_t word = lo == hi ? lo << 16 : (hi << 16) | 1u;
+    return __builtin_bit_cast(float, fabsf(m) + d <= 1.4901161e-8f ? 0u : word);
+}
+// The exact logits of the 16 x 16 block at (t0, e0) whose row or column is unknown (bits of badx, badw), by all WAVES
+// waves of a workgroup: each sums its K / WAVES of the block on the float64 matrix cores (router_gemm_f64_kernel's
+// layouts), the waves' sums are added in LDS. Tokens that are all so cost the float64 GEMM's time (T = 8192: 0.6 ms); one
+// row among others adds 10 us to a call of T = 64 and 70 to one of 8192. (Independent chains or the next loads issued
+// ahead gained nothing.)
+template <int WAVES>
+__device__ __forceinline__ void exact_block(const uint16_t* __restrict__ x, int64_t x_stride,
+                                            const uint16_t* __restrict__ w, int T, int K, int E, int t0, int e0,
+                                            uint32_t badx, uint32_t badw, int wv, double (*ds)[256],
+                                            float* __restrict__ bounds) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int kr = K / WAVES, kq = kr >> 2;                          // kq: a multiple of 16
+    const uint16_t* xp = x + (size_t)min(t0 + r, T - 1) * x_stride + wv * kr + g * kq;
+    const uint16_t* wp = w + (size_t)min(e0 + r, E - 1) * K + wv * kr + g * kq;
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int k = 0; k < kq; k += 16) {
+        u32x4 a[2], b[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            a[h] = *reinterpret_cast<const u32x4*>(xp + k + 8 * h);
+            b[h] = *reinterpret_cast<const u32x4*>(wp + k + 8 * h);
+        }
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const uint32_t av = a[q >> 3][(q >> 1) & 3], bv = b[q >> 3][(q >> 1) & 3], m = 0xFFFF0000u;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                (double)__builtin_bit_cast(float, (q & 1) ? av & m : av << 16),
+                (double)__builtin_bit_cast(float, (q & 1) ? bv & m : bv << 16), acc, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) ds[wv][(g + 4 * v) * 16 + r] = acc[v];
+    __syncthreads();
+    if (threadIdx.x < 256) {
+        const int row = (int)threadIdx.x >> 4, col = (int)threadIdx.x & 15;
+        double dot = ds[0][threadIdx.x];
+#pragma unroll
+        for (int v = 1; v < WAVES; ++v) dot += ds[v][threadIdx.x];
+        if (((badx >> row | badw >> col) & 1u) && t0 + row < T && e0 + col < E)
+            bounds[(size_t)(t0 + row) * E + e0 + col] = router_round(dot);
+    }
+    __syncthreads();                                                 // ds is free again
 }
 
 // 16 tokens x 16 experts per workgroup, its eight waves an eighth of K each: a small call is bound by the latency of its
@@ -236,6 +287,7 @@ __global__ __launch_bounds__(64 * RB_WAVES) void router_bound_kernel(const uint1
                                                                      const uint16_t* __restrict__ w, int T, int K,
                                                                      int E, float* __restrict__ bounds) {
     __shared__ float cs[RB_WAVES][16 * 16], nx[RB_WAVES][16], nw[RB_WAVES][16];
+    __shared__ double ds[RB_WAVES][16 * 16];
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tiles_e = (E + 15) / 16;
@@ -280,16 +332,22 @@ __global__ __launch_bounds__(64 * RB_WAVES) void router_bound_kernel(const uint1
 #pragma unroll
     for (int q = 0; q < 4; ++q) cs[wv][(4 * g + q) * 16 + r] = tot[q];   // D: column lane % 16, row 4 g + q
     __syncthreads();
-    if (threadIdx.x >= 256) return;
-    const int row = (int)threadIdx.x >> 4, col = (int)threadIdx.x & 15;
-    float s = cs[0][threadIdx.x], x2 = nx[0][row], w2 = nw[0][col];
+    const int row = ((int)threadIdx.x >> 4) & 15, col = (int)threadIdx.x & 15;
+    float x2 = nx[0][row], w2 = nw[0][col], n2 = (g & 1) ? nw[0][r] : nx[0][r];
 #pragma unroll
     for (int v = 1; v < RB_WAVES; ++v) {
-        s += cs[v][threadIdx.x];
         x2 += nx[v][row];
         w2 += nw[v][col];
+        n2 += (g & 1) ? nw[v][r] : nx[v][r];
     }
-    if (t0 + row < T && e0 + col < E) bounds[(size_t)(t0 + row) * E + e0 + col] = bound_word(s, x2, w2, K);
+    if (threadIdx.x < 256 && t0 + row < T && e0 + col < E && !norm_unknown(x2) && !norm_unknown(w2)) {
+        float s = cs[0][threadIdx.x];
+#pragma unroll
+        for (int v = 1; v < RB_WAVES; ++v) s += cs[v][threadIdx.x];
+        bounds[(size_t)(t0 + row) * E + e0 + col] = bound_word(s, x2, w2, K);
+    }
+    const uint32_t bad = (uint32_t)__ballot(norm_unknown(n2));        // rows, then columns (the same in every wave)
+    if (bad) exact_block<RB_WAVES>(x, x_stride, w, T, K, E, t0, e0, bad & 0xFFFFu, bad >> 16, wv, ds, bounds);
 }
 
 // 64 tokens x 96 experts per workgroup (288 experts are three such tiles), four waves: wave (b, q) takes token block b of
@@ -385,17 +443,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void r
 #pragma unroll
             for (int q = 0; q < 16; ++q) cs[((b * 3 + n) * 32 + 8 * (q >> 2) + 4 * h + (q & 3)) * 32 + r] = tot[n][q];
     __syncthreads();
-    if (q2 == 1) return;
+    if (q2 == 0)
 #pragma unroll
-    for (int n = 0; n < 3; ++n) {
-        const int e = e0 + 32 * n + r;
-        const float w2 = nw[32 * n + r] + nw[RBB_EXP + 32 * n + r];
+        for (int n = 0; n < 3; ++n) {
+            const int e = e0 + 32 * n + r;
+            const float w2 = nw[32 * n + r] + nw[RBB_EXP + 32 * n + r];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int row = 8 * (q >> 2) + 4 * h + (q & 3), t = 32 * b + row;
-            const float s = tot[n][q] + cs[((b * 3 + n) * 32 + row) * 32 + r];
-            if (t0 + t < T && e < E) bounds[(size_t)(t0 + t) * E + e] = bound_word(s, nx[t] + nx[RBB_TOK + t], w2, K);
+            for (int q = 0; q < 16; ++q) {
+                const int row = 8 * (q >> 2) + 4 * h + (q & 3), t = 32 * b + row;
+                const float s = tot[n][q] + cs[((b * 3 + n) * 32 + row) * 32 + r], x2 = nx[t] + nx[RBB_TOK + t];
+                if (t0 + t < T && e < E && !norm_unknown(x2) && !norm_unknown(w2))
+                    bounds[(size_t)(t0 + t) * E + e] = bound_word(s, x2, w2, K);
+            }
         }
+    // the blocks of an unknown row or column, one after another by the whole workgroup (the same in every wave)
+    const int e2 = RBB_EXP - 32 + (lane & 31);
+    const uint64_t badx = __ballot(norm_unknown(nx[lane] + nx[RBB_TOK + lane]));
+    const uint64_t badw = __ballot(norm_unknown(nw[lane] + nw[RBB_EXP + lane]));
+    const uint32_t badw2 = (uint32_t)__ballot(norm_unknown(nw[e2] + nw[RBB_EXP + e2]));
+    if ((badx | badw | badw2) == 0) return;
+    double(*ds)[256] = reinterpret_cast<double(*)[256]>(lds + 32768);   // (past cs and the norms)
+    for (int u = 0; u < (RBB_TOK / 16) * (RBB_EXP / 16); ++u) {
+        const int tb = u / (RBB_EXP / 16), eb = u % (RBB_EXP / 16);
+        const uint32_t bx = (uint32_t)(badx >> (16 * tb)) & 0xFFFFu;
+        const uint32_t bw = (eb < 4 ? (uint32_t)(badw >> (16 * eb)) : badw2 >> (16 * (eb - 4))) & 0xFFFFu;
+        if (bx | bw) exact_block<4>(x, x_stride, w, T, K, E, t0 + 16 * tb, e0 + 16 * eb, bx, bw, wv, ds, bounds);
     }
 }
 // Tokens from which the big tiles win (whole layer, 288 experts x 4096, big against small tiles: T = 300 621 / 607 us,

@@ -54,3 +54,69 @@ def test_picks_hard_operands(cuda, kind):
     elif kind == "nan":
         x[3, 5], x[4, 6], x[5, 7], w[9, 5] = float("nan"), float("inf"), -float("inf"), 0.0
     _check(cuda, T, E, K, 8, x, w, b)
+
+
+def _operands(cuda, kind, T, E, K):
+    from mi355moe import synthetic
+    w, b = synthetic.router(E, K, seed=17, device=cuda)
+    x = synthetic.activations(T, K, seed=18, device=cuda)
+    g = torch.Generator(device=cuda).manual_seed(19)
+    if kind == "zero":                                # padding: token rows and experts
+        x[::2] = 0
+        w[1::3] = 0
+    elif kind == "tiny":                              # squares below the fp32 range; scores all 0.5
+        x[::2] *= 1e-22
+        w[1::3] *= 1e-20
+    elif kind == "huge":                              # norms past the fp32 range, half of the tokens and one expert
+        x[::2] *= 1e25
+        w[3] *= 1e30
+    elif kind == "nan":
+        x[T - 2, 5], x[7, K - 1], w[E - 1, 3] = float("nan"), float("inf"), float("nan")
+    elif kind == "cancel":                            # sums far below the norms: whole and in every pair of products
+        x[:, 1::2] = x[:, ::2]
+        w[:, 1::2] = -w[:, ::2]
+        w += (torch.randn(E, K, generator=g, device=cuda) * 1e-4).to(w.dtype)
+    elif kind == "wide":                              # exponents over 24 binades
+        x *= torch.exp2(torch.rand(T, K, generator=g, device=cuda) * 24 - 12).to(x.dtype)
+        w *= torch.exp2(torch.rand(E, K, generator=g, device=cuda) * 24 - 12).to(w.dtype)
+    elif kind == "outliers":                          # a few large channels that the router weights down
+        x[:, ::512] *= 300.0
+        w[:, ::512] *= 0.003
+    return x, w, b
+
+
+# the small tiles, and from 1024 tokens the large ones; up to 320 experts and more (another top-k); partial tiles
+@pytest.mark.parametrize("T,E,K", [(33, 40, 1024), (70, 288, 4096), (1030, 100, 512), (1100, 400, 2048)])
+@pytest.mark.parametrize("kind", ["plain", "zero", "tiny", "huge", "nan", "cancel", "wide", "outliers"])
+def test_bound_words(cuda, kind, T, E, K):
+    """Every stored word against the exact logit: exact ones are it (or 0 for one within 2^-26, whose score is 0.5 too),
+    upper bounds are not below it, and rows that are zero, tiny, not finite or too large for fp32 norms have exact words
+    only. The picks and weights are those of the exact logits."""
+    import ctypes
+
+    from mi355moe import _lib, ops, synthetic
+    print(f"bound words {kind} T={T} E={E} K={K}", flush=True)
+    topk = 8
+    x, w, b = _operands(cuda, kind, T, E, K)
+    ex = synthetic.exl3_layer(2, K, 128, seed=3, device=cuda)
+    lg = ops.router_logits(x, w)
+    ids, wts = ops.router_topk(lg, topk, bias=b, routed_scale=2.5)
+    _, gi, gw = ops.moe_layer(ex, x, router_w=w, topk=topk, bias=b, routed_scale=2.5, return_picks=True)
+    # the call's router scratch follows the experts' part of the workspace
+    desc = ctypes.byref(ex.desc)
+    base = _lib.lib().mi355moe_moe_workspace_bytes_path(desc, T, topk, _lib.PATH_AUTO)
+    ws = ops.workspace(cuda, _lib.lib().mi355moe_moe_layer_workspace_bytes(desc, T, topk, E))
+    off = (base + 255) // 256 * 256
+    words = ws[off:off + 4 * T * E].view(torch.int32).view(T, E).clone()
+    torch.cuda.synchronize()
+    low, val = words & 0xFFFF, (words & -65536).view(torch.float32)
+    assert ((low == 0) | (low == 1)).all()
+    small = lg.abs() <= 2.0 ** -26
+    ok = torch.where(low == 0, (val == lg) | (small & (val == 0)) | (val.isnan() & lg.isnan()), val >= lg)
+    assert ok.all(), (kind, int((~ok).sum()), lg[~ok][:4], val[~ok][:4])
+    known = {"zero": (slice(None, None, 2), slice(1, None, 3)), "tiny": (slice(None, None, 2), slice(1, None, 3)),
+             "huge": (slice(None, None, 2), 3), "nan": ([T - 2, 7], E - 1)}.get(kind)
+    if known:
+        assert (low[known[0]] == 0).all() and (low[:, known[1]] == 0).all()
+    assert torch.equal(ids, gi)
+    assert torch.equal(wts.view(torch.int32), gw.view(torch.int32))
