@@ -1482,7 +1482,9 @@ int launch_router_picks(const uint16_t* x, int64_t x_stride, const uint16_t* w, 
                         const float* bias, int topk, float scale, int renorm, int32_t* ids, float* wts,
                         hipStream_t st) {
     if (E > TOPK_MAX_E || topk > TOPK_MAX_K || K % 512 || T <= 0) return -1;
-    if (T >= RB_BIG_T) {
+    // (LDS DMA of 16 bytes a lane wants 16-byte addresses; an x with another base was always taken, by ordinary loads)
+    const bool dma_ok = (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
+    if (T >= RB_BIG_T && dma_ok) {
         const dim3 g((unsigned)(((T + RBB_TOK - 1) / RBB_TOK) * ((E + RBB_EXP - 1) / RBB_EXP)));
         hipLaunchKernelGGL(router_bound_big_kernel, g, dim3(256), 0, st, x, x_stride, w, T, K, E, bounds);
     } else {

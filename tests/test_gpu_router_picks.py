@@ -120,3 +120,16 @@ def test_bound_words(cuda, kind, T, E, K):
         assert (low[known[0]] == 0).all() and (low[:, known[1]] == 0).all()
     assert torch.equal(ids, gi)
     assert torch.equal(wts.view(torch.int32), gw.view(torch.int32))
+
+
+@pytest.mark.parametrize("T", [40, 1030])
+def test_picks_of_unaligned_rows(cuda, T):
+    """x a column range of a wider buffer, 8 bytes past a 16-byte address (its row stride is a multiple of 16 bytes)."""
+    from mi355moe import synthetic
+    print(f"picks of unaligned rows T={T}", flush=True)
+    E, K = 100, 1024
+    w, b = synthetic.router(E, K, seed=25, device=cuda)
+    wide = synthetic.activations(T, K + 64, seed=26, device=cuda)
+    x = wide[:, 4:4 + K]
+    assert x.data_ptr() % 16 == 8
+    _check(cuda, T, E, K, 4, x, w, b)
