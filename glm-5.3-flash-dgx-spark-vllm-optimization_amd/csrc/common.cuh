@@ -303,7 +303,8 @@ __device__ __forceinline__ const T* uniform_ptr(const T* p) {
     return reinterpret_cast<const T*>((uintptr_t)u);
 }
 // The same with a wave-uniform base and a 32-bit byte offset per lane (no 64-bit address arithmetic on the VALU);
-// COH: as dma16_coh below.
+// COH: a device-coherent load (agent scope, sc1: the data comes from the device coherence point, not from a line another
+// XCD's stores left stale in this CU's or XCD's caches).
 template <bool COH = false>
 __device__ __forceinline__ void dma16_base(const void* base, uint32_t off_lane, unsigned char* lds_wave) {
     const uint32_t m0 = (uint32_t)(uintptr_t)lds_wave;
@@ -320,13 +321,6 @@ __device__ __forceinline__ void dma16_base(const void* base, uint32_t off_lane, 
 __device__ __forceinline__ void dma16_nt(const void* src_lane, unsigned char* lds_wave) {
     const uint32_t m0 = (uint32_t)(uintptr_t)lds_wave;
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(m0), "v"(src_lane)
-                 : "memory", "m0");
-}
-// The same as a device-coherent load (agent scope, sc1: the data comes from the device coherence point, not from a
-// line another XCD's stores left stale in this CU's or XCD's caches).
-__device__ __forceinline__ void dma16_coh(const void* src_lane, unsigned char* lds_wave) {
-    const uint32_t m0 = (uint32_t)(uintptr_t)lds_wave;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off sc1" ::"s"(m0), "v"(src_lane)
                  : "memory", "m0");
 }
 // Device-coherent 16-byte accesses (sc1: agent scope, served by the device coherence point, the cache policy

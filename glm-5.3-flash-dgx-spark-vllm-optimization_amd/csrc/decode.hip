@@ -429,7 +429,8 @@ __device__ __forceinline__ void gateup_tile(const DecodeArgs& a, int cb, int s, 
     }
     __builtin_amdgcn_sched_barrier(0);
 
-    // the first batch in straight-line code (so its wait leaves the prefetch in flight), then any further batches
+    // the first batch in straight-line code (so its wait leaves the prefetch in flight), then any further batches; the DMA
+    // is waited for together with the prefetch
     if constexpr (PRE) {
         if (dma) {
             WAIT_VM(0);                                              // this wave's DMA has landed

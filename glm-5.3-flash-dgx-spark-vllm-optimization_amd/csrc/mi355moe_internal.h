@@ -9,7 +9,6 @@ enum DType { DT_F32 = 0, DT_F16 = 1, DT_BF16 = 2 };
 
 constexpr int ROUTE_SMALL_MAX_P = 1024;   // pairs the one-block permutation handles
 
-// Permutation of P = T * topk routed pairs into expert order.
 // Rotated token rows for a layer whose experts share one w13 suh: out[t][k] = fp16(H(fp16(x[t] * suh)) * r), fp16, the
 // columns of every 16-group in the staged order 0, 1, 8, 9, 2, 3, ... (out == nullptr: none)
 struct RotateArgs {
@@ -21,6 +20,7 @@ struct RotateArgs {
     uint16_t* out;          // [T][K]
 };
 
+// Permutation of P = T * topk routed pairs into expert order.
 struct RouteArgs {
     const void* ids;        // [P] int32 or int64 router ids
     int ids64;
@@ -94,7 +94,7 @@ struct DecodeArgs {
     int kch_gu, kch_dn;     // chunk length (K elements for gate/up, N elements for down)
     int rmax;               // rows per segment (<= 16)
     int shared_suh;         // gate and up share one input rotation (one staged copy)
-    int lds_gu;             // LDS bytes the gate/up passes are planned for (set by launch_decode)
+    int lds_gu;             // LDS bytes the gate/up passes are planned for (set by launch_decode: DECODE_LDS_MAX or _ONE)
     float limit;
     // workspace
     float* zg;              // [K / kch_gu][2][P][N] partial sums, slot = the fragment's first chunk
@@ -290,8 +290,9 @@ struct Fp8Args {
 constexpr int FP8_TM = 64;   // rows per segment (two 32-row MFMA tiles)
 // Calls of up to FP8_FEW_T tokens take segments of FP8_FEW rows and kernels that stage only those: 17 instead of 24 KB per
 // stage, so three workgroups (96 KB of weights in flight) share a CU instead of two (64 KB). An expert with more rows is
-// read once per segment, at most twice here.
-// T = 12, 288 experts, hidden 4096, intermediate 1024: 235 -> 188 us.
+// read once per segment, at most twice here. us with 64- / 8-row segments, top-8, hidden 4096, intermediate 1024: 288
+// experts T = 1 60 / 45, 4 104 / 87, 12 235 / 188, 16 296 / 240, Zipf routing T = 8 137 / 98, 16 174 / 139; 16 experts
+// (8 rows each at T = 16, some in two segments) T = 4 74 / 62, 16 75 / 71; 8 experts (16 rows, two segments) T = 16 65 / 55.
 constexpr int FP8_FEW = 8, FP8_FEW_T = 16;
 constexpr int fp8_seg_rows(int64_t tokens) { return tokens <= FP8_FEW_T ? FP8_FEW : FP8_TM; }
 // kernels: bit 0 quantize inputs, bit 1 gate/up, bit 2 down-input quantization + down, bit 3 slot-order combine

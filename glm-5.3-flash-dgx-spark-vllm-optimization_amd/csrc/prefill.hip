@@ -437,14 +437,6 @@ __device__ __forceinline__ int pf_swz(int R) { return PF_RB == 64 ? (R >> 2) & 3
 // w[0] = word wp - 1, w[1] = word wp, w[2] = word wp + 1. Pair p (0..7) of the lane: word wp (p < 4) or wp + 1,
 // states 2 (p % 4) and 2 (p % 4) + 1 of that word (decode_word's order); the operand of column 16t + c is pairs
 // 0, 1, 4, 5 (k slots 8h .. 8h + 7) and that of column 16t + c + 8 is pairs 2, 3, 6, 7.
-__device__ __forceinline__ void pf_load_words(const unsigned char* wk, int lane, uint32_t (&w)[3]) {
-    const int n = lane & 31, wp = 4 * (n & 7) + 2 * (lane >> 5);
-    const unsigned char* tile = wk + (n >> 3) * 128;
-    const uint2 v = *reinterpret_cast<const uint2*>(tile + 4 * wp);
-    w[0] = *reinterpret_cast<const uint32_t*>(tile + 4 * ((wp + 31) & 31));
-    w[1] = v.x;
-    w[2] = v.y;
-}
 // The pair's decode in two halves (software-pipelined across MFMA pairs by the GEMM loop): pf_pair_products =
 // the two states times MCG_MUL, pf_pair_values = mask, flip and the fp16 sums.
 struct PfPair {
@@ -1108,7 +1100,7 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 // ------------------------------------------------------------------------------------------------ one-launch schedule
 
 // Every gate/up and down tile of a call in one launch of one workgroup per CU (256-row tiles; two per CU for the
-// 128-row and three for the 64-row part tiles, KIND below). The segments are dealt to eight ticket queues (segment s to queue s % 8, as the separate launches deal them to the
+// 128-row and two or three for the 64-row part tiles, KIND below). The segments are dealt to eight ticket queues (segment s to queue s % 8, as the separate launches deal them to the
 // XCDs), each ordered by pf_sched_item over its own segments; a workgroup takes tickets from its own XCD's queue
 // (the XCC_ID register), so a segment's column blocks share that XCD's L2 for their A rows, and once that queue is
 // empty from the other queues in turn. A gate/up item stores its h2 rows device-coherent (written through to the
@@ -1221,8 +1213,13 @@ __global__ __launch_bounds__(PF_THREADS, 1) void pf_sched_kernel(PrefillArgs a) 
     extern __shared__ __align__(16) unsigned char smem[];
     pf_sched_body<MODE, PF_LARGE>(a, smem);
 }
+// Workgroups per CU of the part tiles: three of 64 rows with E3's numerics, two with e4m3's, whose longer decode keeps the
+// VALU busy with two and (where the down input is quantised in the launch) spills within the 168 registers of three: calls
+// on 64-row tiles were 3 - 5 % slower on average with three, and Zipf ones up to 18 % (96 experts, hidden 4096,
+// intermediate 512, top-8, T = 256 Zipf 279 / 245 us).
+constexpr int pf_sched_part_cu(int mode, int kind) { return kind == PF_SMALL && mode == PF_SCHED_E3 ? 3 : 2; }
 template <int MODE, int KIND>
-__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(KIND == PF_SMALL ? 3 : 2))) void pf_sched_part_kernel(
+__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(pf_sched_part_cu(MODE, KIND)))) void pf_sched_part_kernel(
     PrefillArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     pf_sched_body<MODE, KIND>(a, smem);
@@ -1644,7 +1641,10 @@ int prefill_setup() {
 //   T = 2048 (57 rows):             mid 870 / 976, small 880 / 1036 (T = 2000), 256-row tiles about 1110 / 1366
 //   T = 4096 (~114 rows):           mid 29 % / 21 % faster than the 256-row tiles
 //   T = 6144 (~171 rows):           mid 4 % slower; T = 8192 (~228 rows): mid 8 % slower (Zipf: mid 4 % faster).
-// Hence: P <= 36 n: small; P <= 128 n: mid; larger calls: the 256-row kernels. P is the pairs expected on this call's
+// Hence: P <= 36 n: small; P <= 128 n: mid; larger calls: the 256-row kernels. With e4m3 also small where all 64-row
+// gate/up tiles of up to 128 rows per expert have a slot at once, two per CU: few mid tiles leave CUs idle (96 experts,
+// hidden 4096, intermediate 256, e4m3 small / mid: 58 rows per expert 208 / 229, Zipf 227 / 256, 100 rows 262 / 283, Zipf
+// 266 / 291; intermediate 512, 75 rows, more tiles than slots: 351 / 297). P is the pairs expected on this call's
 // experts: with an expert map only the share n / n_global of the routed ones (144 of 288 experts, T = 4289, Zipf
 // routing, 119 rows per expert: mid 823 us, 256-row tiles 931). "hybrid" splits a call by segment size (segments of at
 // most PF_SMALL_ROWS rows on the small tiles, larger ones on the 256-row tiles). The environment variable
@@ -1661,6 +1661,8 @@ static int pf_tiles(const PrefillArgs& a) {
     if (a.n <= 0) return PF_TILES_LARGE;
     const int64_t P = a.pairs_local > 0 ? a.pairs_local : a.P, n = a.n;
     if (P <= 36 * n) return PF_TILES_SMALL;
+    if (a.e4m3 && P <= 128 * n && n * (a.N >> 7) * ((P + 64 * n - 1) / (64 * n)) <= 2 * pf_device_cus())
+        return PF_TILES_SMALL;
     return P <= 128 * n ? PF_TILES_MID : PF_TILES_LARGE;
 }
 
@@ -1702,10 +1704,10 @@ int launch_prefill(const PrefillArgs& a0, hipStream_t st, int kernels) {
     if (sched) {
         a.small_rows = 0;
         const int parts = tiles == PF_TILES_SMALL ? 4 : tiles == PF_TILES_MID ? 2 : 1;
-        const int per_cu = parts > 2 ? 3 : parts > 1 ? 2 : 1;
+        const int mode = !f8 ? PF_SCHED_E3 : a.down16 ? PF_SCHED_E4M3_16 : PF_SCHED_E4M3;
+        const int per_cu = parts == 1 ? 1 : pf_sched_part_cu(mode, parts > 2 ? PF_SMALL : PF_MID);
         const int64_t items = (int64_t)std::max(a.S_cap, 0) * parts * ((a.N >> 7) + (a.K >> 8));
         const dim3 grid((unsigned)std::min<int64_t>((int64_t)per_cu * pf_device_cus(), items)), blk(PF_THREADS);
-        const int mode = !f8 ? 0 : a.down16 ? 1 : 2;
         if (grid.x > 0) {
             if (parts == 1) {
                 if (mode == 0) hipLaunchKernelGGL(pf_sched_kernel<PF_SCHED_E3>, grid, blk, PF_LDS, st, a);

@@ -190,9 +190,11 @@ __global__ __launch_bounds__(256) void router_gemm_f64_kernel(const uint16_t* __
 constexpr int RG_MIN_T = 256;   // from this many tokens the MFMA GEMM beats the GEMV kernel
 
 // Router logits for the top-k alone (router_bound_kernel, router_bound_big_kernel): products on the bf16 matrix cores
-// with fp32 sums, a rigorous bound on their error, and for every logit either its value (the bound leaves one bf16
-// value possible) or an upper bound of it; the top-k then takes the exact dot product of a candidate only when its
-// upper bound wins a round (topk_wave, LAZY): about one per token. The picks and weights are those of the exact logits.
+// with fp32 sums, a bound on their error, and for every logit either its value (the bound leaves one bf16 value possible)
+// or an upper bound of it; the top-k then takes the exact dot product of a candidate only when its upper bound wins a
+// round (topk_wave, LAZY): about one per token (Gaussian operands; with a few large channels that the router weights
+// down, which widen the bound, some eight: T = 8192 145 us instead of 95). The picks and weights are those of the exact
+// logits.
 //
 // Error bound: a sum runs as chains of 64 products from zero, each chain added to an fp32 total (and the totals of a
 // workgroup's K ranges added in order). However the matrix core orders, aligns and truncates, an addend of an MFMA
@@ -570,7 +572,10 @@ __device__ void build_segments(const int* cnt, const int* start, int n, int R, i
 
 // Rotated token rows (RotateArgs), in tasks of one wave: token t, four 128-blocks (16 lanes per block, 8 consecutive
 // elements per lane). Wave w of nw takes tasks w, w + nw, ... The product with r is rounded to fp32 before fp16 (as the
-// oracle has it): without the barrier the compiler fuses the two in some call sites and not in others.
+// oracle has it): without the barrier the compiler fuses the two in some call sites and not in others. The workgroups'
+// own rotation (stage8_store in the gate/up kernel: calls of up to 4 tokens, split K ranges, layers of several suh) has
+// no such barrier, so there a staged value on a rounding boundary may differ by one fp16 ulp; errors against float64
+// are the same.
 __device__ void rotate_tasks(const RotateArgs& a, int w, int nw) {
     const int lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
     const int nb = a.K >> 7, np = (nb + 3) >> 2;

@@ -134,3 +134,25 @@ def test_e4m3_trellis_full_size_token_sample(cuda):
          f"elements outside rtol 2e-2 / atol 1e-3")
     assert r <= 1e-3, r
     assert r4 <= 1e-5 and np.allclose(got, y4, rtol=2e-2, atol=1e-3), r4
+
+
+@pytest.mark.parametrize("down16", [False, True])
+@pytest.mark.parametrize("T", [72, 73, 128, 129, 256, 257])
+def test_e4m3_tile_kinds(cuda, monkeypatch, T, down16):
+    """Sizes around the tile rule's lines (36, 64 and 128 pairs per expert): the call's own choice and each part tile are
+    bit-identical to the 256-row tiles."""
+    from mi355moe import ops, synthetic
+    n, K, N, topk = 4, 512, 256, 2
+    _say(f"e4m3 tile kinds T={T} down16={down16}")
+    ex = synthetic.calibrated_layer(n, K, N, seed=61, device=cuda, uniform_suh=True)
+    x = synthetic.activations(T, K, seed=62, device=cuda)
+    ids = synthetic.random_ids(T, n, topk, seed=63, device=cuda)
+    w = synthetic.softmax_weights(T, topk, seed=64, device=cuda)
+    out = {}
+    for tiles in ("large", "auto", "small", "mid"):
+        monkeypatch.setenv("MI355MOE_PREFILL_TILES", tiles)
+        out[tiles] = ops.moe_forward_ids_e4m3(ex, x, ids, w, limit=10.0, out_dtype=torch.float32, down16=down16)
+    torch.cuda.synchronize()
+    assert torch.isfinite(out["large"]).all()
+    for tiles in ("auto", "small", "mid"):
+        assert torch.equal(out[tiles], out["large"]), tiles
