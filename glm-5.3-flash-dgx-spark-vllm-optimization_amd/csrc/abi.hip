@@ -106,7 +106,7 @@ double expected_experts(double T, int64_t topk, int64_t n, int64_t total) {
 // faster on average, 8 of them 3 to 8 % slower; planned for uniform routing alone (129 workgroups of the local experts)
 // 510 of them were 3 to 28 % slower.
 bool splits_do(int64_t h, double wu, double ws, double keep, bool tail) {
-    constexpr double CUS = 256.0, SPILL = 350.0;
+    constexpr double CUS = 256.5, SPILL = 350.0;                     // (256: one round, whatever pow rounds to)
     return ws * (double)h >= keep && !(tail && wu * (double)h > CUS && wu * (double)h <= SPILL);
 }
 constexpr double SPLIT_KEEP = 144.0;   // 9 of 16 CUs
