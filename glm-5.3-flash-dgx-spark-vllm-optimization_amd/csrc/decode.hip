@@ -956,7 +956,8 @@ int launch_rot_in(const void* x, int xdt, int64_t x_stride, const int* tok, cons
 }
 
 size_t decode_staged_gateup(int rmax, int kr, int shared_suh) {
-    return (size_t)std::max(gateup_staged(rmax, kr, shared_suh != 0), gateup_staged(std::min(rmax, DUP_ROWS), kr, shared_suh != 0));
+    return (size_t)std::max(gateup_staged(rmax, kr, shared_suh != 0),
+                            gateup_staged(std::min(rmax, DUP_ROWS), kr, shared_suh != 0));
 }
 size_t decode_lds_gateup(int rmax, int kr, int shared_suh, size_t limit) {
     // the largest staging of any segment of up to rmax rows that fits `limit` (0: some segment fits no pass)

@@ -234,10 +234,11 @@ int launch_prefill(const PrefillArgs& a, hipStream_t st, int kernels);
 // A call over caller-built row tables (rows a.P = rows_cap, segments a.seg_* / a.nseg, chunk a.chunk / a.nchunks):
 // the rows the live segments cover are marked in pe (their segment's expert, or a.row_expert[r]), every other row -1;
 // then optionally e4m3 code rows widened into the GEMMs' fp16 staging (a8 -> a8_dst: every row < a8_rows, or only the
-// marked ones, with a8_tok row r from a8 row tok32[r]), launch_prefill's `kernels` over the marked rows, and with tokens > 0 every token's marked rows
-// (row_token) summed in row order and ADDED to out (fp32 or bf16 [tokens][K], row stride a.out_stride) with the row
-// weights a.w32 (fp32) or a.w16 (fp16). tok32 (optional): [P] the rows' tokens as int32 (outside [0, tokens): 0), for
-// token-row A operands. cnt [tokens], list [tokens][PF_ROWS_PER_TOKEN] and pe [P] are scratch.
+// marked ones, with a8_tok row r from a8 row tok32[r]), launch_prefill's `kernels` over the marked rows, and with
+// tokens > 0 every token's marked rows (row_token) summed in row order and ADDED to out (fp32 or bf16 [tokens][K], row
+// stride a.out_stride) with the row weights a.w32 (fp32) or a.w16 (fp16). tok32 (optional): [P] the rows' tokens as
+// int32 (outside [0, tokens): 0), for token-row A operands. cnt [tokens], list [tokens][PF_ROWS_PER_TOKEN] and pe [P]
+// are scratch.
 struct RowsPlan {
     int* pe;
     const int64_t* row_token;

@@ -1100,10 +1100,10 @@ __global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 // ------------------------------------------------------------------------------------------------ one-launch schedule
 
 // Every gate/up and down tile of a call in one launch of one workgroup per CU (256-row tiles; two per CU for the
-// 128-row and two or three for the 64-row part tiles, KIND below). The segments are dealt to eight ticket queues (segment s to queue s % 8, as the separate launches deal them to the
-// XCDs), each ordered by pf_sched_item over its own segments; a workgroup takes tickets from its own XCD's queue
-// (the XCC_ID register), so a segment's column blocks share that XCD's L2 for their A rows, and once that queue is
-// empty from the other queues in turn. A gate/up item stores its h2 rows device-coherent (written through to the
+// 128-row and two or three for the 64-row part tiles, KIND below). The segments are dealt to eight ticket queues
+// (segment s to queue s % 8, as the separate launches deal them to the XCDs), each ordered by pf_sched_item over its own
+// segments; a workgroup takes tickets from its own XCD's queue (the XCC_ID register), so a segment's column blocks share
+// that XCD's L2 for their A rows, and once that queue is empty from the other queues in turn. A gate/up item stores its h2 rows device-coherent (written through to the
 // device coherence point, so no L2 write-back fence is needed), and once every wave's stores have completed
 // (s_waitcnt, then a barrier) one lane raises the segment's count. A down item waits until the count reaches the
 // segment's ncg gate/up items (one lane polls with agent-scope atomic loads, sleeping between polls) and loads the
@@ -1219,8 +1219,8 @@ __global__ __launch_bounds__(PF_THREADS, 1) void pf_sched_kernel(PrefillArgs a) 
 // intermediate 512, top-8, T = 256 Zipf 279 / 245 us).
 constexpr int pf_sched_part_cu(int mode, int kind) { return kind == PF_SMALL && mode == PF_SCHED_E3 ? 3 : 2; }
 template <int MODE, int KIND>
-__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(pf_sched_part_cu(MODE, KIND)))) void pf_sched_part_kernel(
-    PrefillArgs a) {
+__global__ __launch_bounds__(PF_THREADS) __attribute__((amdgpu_waves_per_eu(pf_sched_part_cu(MODE, KIND)))) void
+pf_sched_part_kernel(PrefillArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     pf_sched_body<MODE, KIND>(a, smem);
 }
